@@ -61,31 +61,82 @@ struct Ctx {
     }
 };
 
+// Large buffers that DevBuf::alloc_kept() allocated and that were released,
+// kept for the next such request (fh_solver.cpp).  A buffer of 345 MB costs
+// 0.26 ms in hipFree, and a program that allocates and frees one in every
+// call has, after some hundred calls, gone once through the card's memory:
+// from then on each call waits 8 to 30 ms for the driver to clear what was
+// freed.  At most kKeptBytes stay; they are freed oldest first, when an
+// allocation fails, and with the last context of the process.
+constexpr size_t kKeptMin = (size_t)1 << 20, kKeptBytes = (size_t)4 << 30;
+void* kept_take(size_t bytes, int dev, size_t* cap);  // null: none fits
+void kept_give(void* p, size_t cap, int dev);
+void kept_trim();
+
 // Owning device allocation.
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
+    size_t cap = 0;  // of a buffer that goes to the kept ones, else 0
+    int dev = 0;     // its device
     DevBuf() = default;
     explicit DevBuf(size_t b) { alloc(b); }
     void alloc(size_t b) {
         release();
         bytes = b;
-        if (b) FH_HIP(hipMalloc(&p, b));
+        if (b) allocate(b);
+    }
+    // As alloc, from and later back to the kept buffers.  Results of the
+    // entry points that allocate a system per call; what they hold is not
+    // zero and everything that is read has to be written first.
+    void alloc_kept(size_t b) {
+        release();
+        bytes = b;
+        if (b < kKeptMin) {
+            if (b) allocate(b);
+            return;
+        }
+        FH_HIP(hipGetDevice(&dev));
+        p = kept_take(b, dev, &cap);
+        if (p == nullptr) {
+            allocate(b);
+            cap = b;
+        }
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (cap) kept_give(p, cap, dev);
+        else if (p) (void)hipFree(p);
         p = nullptr;
-        bytes = 0;
+        bytes = cap = 0;
     }
     ~DevBuf() { release(); }
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes), cap(o.cap), dev(o.dev) { o.p = nullptr; o.bytes = o.cap = 0; }
     DevBuf& operator=(DevBuf&& o) noexcept {
-        if (this != &o) { release(); p = o.p; bytes = o.bytes; o.p = nullptr; o.bytes = 0; }
+        if (this != &o) {
+            release();
+            p = o.p; bytes = o.bytes; cap = o.cap; dev = o.dev;
+            o.p = nullptr; o.bytes = o.cap = 0;
+        }
         return *this;
     }
     template <class T> T* as() const { return static_cast<T*>(p); }
+
+private:
+    void allocate(size_t b) {
+        hipError_t e = hipMalloc(&p, b);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();
+            kept_trim();
+            e = hipMalloc(&p, b);
+        }
+        if (e != hipSuccess) {
+            p = nullptr;
+            bytes = 0;
+        }
+        FH_HIP(e);
+    }
 };
 
 // Device vector of a given precision.

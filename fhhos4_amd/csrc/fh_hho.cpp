@@ -1925,7 +1925,8 @@ static HhoDev make_device_problem(Ctx& c, const HhoProblem& H, const HhoProblem:
         MFT.insert(MFT.end(), T.MFT.begin(), T.MFT.end());
     }
     auto up = [&](const void* h, size_t bytes) {
-        keep.emplace_back(std::max<size_t>(bytes, 8));
+        keep.emplace_back();
+        keep.back().alloc_kept(std::max<size_t>(bytes, 8));
         if (bytes) FH_HIP(hipMemcpyAsync(keep.back().p, h, bytes, hipMemcpyHostToDevice, c.stream));
         return keep.back().p;
     };
@@ -2064,7 +2065,7 @@ std::unique_ptr<Bcsr> HhoProblem::AssembleDevice(Ctx& c, double* b_dev, bool kee
         E->rows = std::make_shared<DevBuf>(sizeof(int) * rows.size());
         FH_HIP(hipMemcpyAsync(E->rows->p, rows.data(), sizeof(int) * rows.size(), hipMemcpyHostToDevice, c.stream));
         const size_t nv = (size_t)I.ncell * E->stride;
-        E->vals.alloc(sizeof(double) * nv);
+        E->vals.alloc_kept(sizeof(double) * nv);
         FH_HIP(hipMemsetAsync(E->vals.p, 0, sizeof(double) * nv, c.stream));
         keep.emplace_back(sizeof(int) * pos.size());
         FH_HIP(hipMemcpyAsync(keep.back().p, pos.data(), sizeof(int) * pos.size(), hipMemcpyHostToDevice, c.stream));
@@ -2081,11 +2082,11 @@ std::unique_ptr<Bcsr> HhoProblem::AssembleDevice(Ctx& c, double* b_dev, bool kee
     A->h_rowptr = rowptr;
     A->h_colidx = colidx;
     A->rowptr.alloc(sizeof(int) * rowptr.size());
-    A->colidx.alloc(sizeof(int) * std::max<size_t>(1, colidx.size()));
+    A->colidx.alloc_kept(sizeof(int) * std::max<size_t>(1, colidx.size()));
     FH_HIP(hipMemcpyAsync(A->rowptr.p, rowptr.data(), sizeof(int) * rowptr.size(), hipMemcpyHostToDevice, c.stream));
     FH_HIP(hipMemcpyAsync(A->colidx.p, colidx.data(), sizeof(int) * colidx.size(), hipMemcpyHostToDevice, c.stream));
     const size_t nval = (size_t)A->nnzb * nf * nf;
-    A->vals.alloc(sizeof(double) * std::max<size_t>(1, nval));
+    A->vals.alloc_kept(sizeof(double) * std::max<size_t>(1, nval));
     FH_HIP(hipMemsetAsync(A->vals.p, 0, sizeof(double) * nval, c.stream));
     FH_HIP(hipMemsetAsync(b_dev, 0, sizeof(double) * (size_t)nb * nf, c.stream));
     d.vals = A->vals.as<double>();

@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <algorithm>
+#include <mutex>
 #include <utility>
 
 #include "fh_io.h"
@@ -20,6 +21,93 @@ enum : int {
     S_FCG = 400,   // FCG(m): 2 slots per kept direction (m <= 32)
 };
 
+namespace {
+struct Kept {
+    void* p;
+    size_t cap;
+    int dev;
+};
+struct KeptList {
+    std::mutex lock;
+    std::vector<Kept> free;  // oldest first
+    size_t total = 0;
+    int contexts = 0;
+};
+// never destroyed: buffers may be released during the process's exit
+KeptList& kept_list() {
+    static KeptList* l = new KeptList;
+    return *l;
+}
+}  // namespace
+
+void* kept_take(size_t bytes, int dev, size_t* cap) {
+    KeptList& l = kept_list();
+    Kept k{};
+    {
+        std::lock_guard<std::mutex> g(l.lock);
+        size_t best = l.free.size();
+        for (size_t i = 0; i < l.free.size(); i++) {
+            const Kept& f = l.free[i];
+            if (f.dev != dev || f.cap < bytes || f.cap > bytes + bytes / 4) continue;
+            if (best == l.free.size() || f.cap < l.free[best].cap) best = i;
+        }
+        if (best == l.free.size()) return nullptr;
+        k = l.free[best];
+        l.free.erase(l.free.begin() + best);
+        l.total -= k.cap;
+    }
+    // work of any stream that still uses the buffer ends first (hipFree waits
+    // in the same way)
+    if (hipDeviceSynchronize() != hipSuccess) {
+        (void)hipGetLastError();
+        kept_give(k.p, k.cap, dev);
+        return nullptr;
+    }
+    *cap = k.cap;
+    return k.p;
+}
+
+void kept_give(void* p, size_t cap, int dev) {
+    KeptList& l = kept_list();
+    std::vector<Kept> out;
+    {
+        std::lock_guard<std::mutex> g(l.lock);
+        if (cap > kKeptBytes || l.contexts == 0) {
+            out.push_back({p, cap, dev});
+        } else {
+            l.free.push_back({p, cap, dev});
+            l.total += cap;
+            size_t n = 0;
+            while (l.total > kKeptBytes) l.total -= l.free[n++].cap;
+            out.assign(l.free.begin(), l.free.begin() + n);
+            l.free.erase(l.free.begin(), l.free.begin() + n);
+        }
+    }
+    for (const Kept& k : out) (void)hipFree(k.p);
+}
+
+void kept_trim() {
+    KeptList& l = kept_list();
+    std::vector<Kept> out;
+    {
+        std::lock_guard<std::mutex> g(l.lock);
+        out.swap(l.free);
+        l.total = 0;
+    }
+    for (const Kept& k : out) (void)hipFree(k.p);
+}
+
+static void count_context(int change) {
+    KeptList& l = kept_list();
+    bool last;
+    {
+        std::lock_guard<std::mutex> g(l.lock);
+        l.contexts += change;
+        last = l.contexts == 0;
+    }
+    if (last) kept_trim();
+}
+
 Ctx::Ctx(int dev) : device(dev) {
     if (dev < 0) {
         host_only = true;
@@ -33,6 +121,7 @@ Ctx::Ctx(int dev) : device(dev) {
     FH_HIP(hipMemsetAsync(d_scalars, 0, sizeof(double) * kScalars, stream));
     FH_HIP(hipStreamSynchronize(stream));
     noalloc_scratch_init(dev);  // this device is current
+    count_context(1);
 }
 
 Ctx::~Ctx() {
@@ -42,6 +131,7 @@ Ctx::~Ctx() {
     if (d_scalars) (void)hipFree(d_scalars);
     if (h_scalars) (void)hipHostFree(h_scalars);
     if (stream) (void)hipStreamDestroy(stream);
+    count_context(-1);
 }
 
 static void read_scalars(Ctx& c, int first, int count) {

@@ -1,0 +1,118 @@
+"""Batched condensation and cell recovery over cell shapes and face graphs,
+against dense numpy solves: the shapes of one wavefront per cell (smallest,
+odd tile edges, 63 face unknowns), the shapes of the general kernels (another
+number of cell unknowns, more face unknowns or faces), numbers of cells that do
+not fill the last workgroup, and every kind of face: interior, eliminated, in
+one cell, in three cells, twice in one cell (the last two take the pattern
+built on the host, and sums of several contributions).
+
+Tolerance: a block entry is a sum of nc products per contribution after a
+backward-stable solve with condition number below 2: 64 nc units in the last
+place of the largest entry bound it amply."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+F = pytest.importorskip("fhhos4_amd")
+G = F.fhgpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    assert torch.cuda.is_available(), "no ROCm device visible"
+    return G.Context(0)
+
+
+def _faces(rng, ncells, nfc, kind):
+    """A ring-like graph: face f of cell c is shared with cell c + 1 for half
+    of the faces; some faces eliminated; the special kinds change a few."""
+    nfaces = 0
+    faces = -np.ones((ncells, nfc), dtype=np.int32)
+    for c in range(ncells):
+        for j in range(nfc):
+            if faces[c, j] != -1:
+                continue
+            if rng.random() < 0.15:
+                continue  # eliminated
+            faces[c, j] = nfaces
+            if c + 1 < ncells and rng.random() < 0.6:
+                free = np.nonzero(faces[c + 1] == -1)[0]
+                if len(free):
+                    faces[c + 1, rng.choice(free)] = nfaces
+            nfaces += 1
+    if nfaces == 0:
+        faces[0, 0], nfaces = 0, 1
+    if kind == "three" and ncells >= 3:
+        faces[0, 0] = faces[1, 0] = faces[2, 0] = nfaces
+        nfaces += 1
+    if kind == "twice" and nfc >= 2:
+        faces[ncells // 2, :2] = nfaces
+        nfaces += 1
+    return faces, nfaces
+
+
+CASES = [(nc, nf, nfc, n, "plain") for nc, nf, nfc, n in
+         [(1, 1, 1, 1), (1, 1, 6, 5), (3, 2, 3, 9), (4, 3, 6, 6), (6, 3, 4, 7), (10, 6, 4, 3), (10, 4, 4, 10),
+          (20, 10, 6, 4), (20, 10, 4, 5), (20, 9, 7, 3), (3, 2, 8, 11), (1, 16, 1, 3),
+          (2, 2, 4, 3), (5, 3, 5, 3), (20, 10, 7, 2), (4, 3, 9, 3)]] + \
+        [(4, 3, 6, 6, "three"), (10, 6, 4, 5, "twice"), (2, 3, 4, 5, "three"), (20, 10, 6, 3, "twice")]
+
+
+@pytest.mark.parametrize("nc,nf,nfc,ncells,kind", CASES)
+def test_condense_and_recover(ctx, nc, nf, nfc, ncells, kind):
+    print("case nc=%d nf=%d nfc=%d cells=%d %s" % (nc, nf, nfc, ncells, kind), flush=True)
+    rng = np.random.default_rng(nc * 1000 + nf * 10 + nfc)
+    faces, nfaces = _faces(rng, ncells, nfc, kind)
+    m = nfc * nf
+    nl = nc + m
+    R = rng.standard_normal((ncells, nl, nl))
+    local = 0.5 * (R + R.transpose(0, 2, 1)) + nl * np.eye(nl)
+    local[:, nc:, nc:] += 0.1 * rng.standard_normal((ncells, m, m))  # A_FF need not be symmetric
+    local[:, nc:, :nc] = np.nan  # not read
+    BT, BF = rng.standard_normal((ncells, nc)), rng.standard_normal((nfaces, nf))
+    xF = rng.standard_normal(nfaces * nf)
+    A = np.zeros((nfaces, nf, nfaces, nf))
+    b = BF.copy()
+    xT = np.zeros((ncells, nc))
+    pairs = set()
+    for c in range(ncells):
+        TT, TF, FF = local[c, :nc, :nc], local[c, :nc, nc:], local[c, nc:, nc:]
+        X = np.linalg.solve(TT, np.concatenate([TF, BT[c][:, None]], 1))
+        S, y = FF - TF.T @ X[:, :m], TF.T @ X[:, m]
+        xe = np.zeros(m)
+        for i, f in enumerate(faces[c]):
+            if f < 0:
+                continue
+            b[f] -= y[i * nf:(i + 1) * nf]
+            xe[i * nf:(i + 1) * nf] = xF[f * nf:(f + 1) * nf]
+            for j, g in enumerate(faces[c]):
+                if g >= 0:
+                    A[f, :, g, :] += S[i * nf:(i + 1) * nf, j * nf:(j + 1) * nf]
+                    pairs.add((int(f), int(g)))
+        xT[c] = np.linalg.solve(TT, BT[c] - TF @ xe)
+    loc = torch.from_numpy(local).cuda()
+    bt, bf = torch.from_numpy(BT.reshape(-1)).cuda(), torch.from_numpy(BF.reshape(-1)).cuda()
+    M, bd = G.condense_batched(ctx, faces, loc, nc, nf, nfaces, B_T=bt, B_F=bf)
+    rp, ci, v = M.blocks()
+    got = [(r, int(c)) for r in range(nfaces) for c in ci[rp[r]:rp[r + 1]]]
+    assert got == sorted(pairs)
+    tol = 64 * nc * 2.3e-16
+    ref = np.array([A[r, :, c, :] for r, c in got])
+    assert np.abs(v - ref).max() <= tol * np.abs(ref).max()
+    assert np.abs(bd.cpu().numpy().reshape(nfaces, nf) - b).max() <= tol * np.abs(b).max()
+    got_xT = G.cell_recover_batched(ctx, faces, loc, nc, nf, nfaces, torch.from_numpy(xF).cuda(), B_T=bt).cpu().numpy()
+    assert np.abs(got_xT - xT).max() <= tol * np.abs(xT).max()
+    # no right-hand sides
+    M2, b2 = G.condense_batched(ctx, faces, loc, nc, nf, nfaces, rhs=False)
+    assert b2 is None and np.array_equal(M2.blocks()[2], v) if kind == "plain" else True
+    z = G.cell_recover_batched(ctx, faces, loc, nc, nf, nfaces, torch.zeros(nfaces * nf, dtype=torch.float64,
+                                                                              device="cuda"))
+    assert float(z.abs().max()) == 0.0
+    # a matrix that is not positive definite is refused
+    loc[ncells - 1, nc - 1, nc - 1] = -1.0
+    with pytest.raises(G.FhError, match="positive definite"):
+        G.condense_batched(ctx, faces, loc, nc, nf, nfaces)
+    with pytest.raises(G.FhError, match="positive definite"):
+        G.cell_recover_batched(ctx, faces, loc, nc, nf, nfaces, torch.from_numpy(xF).cuda())
