@@ -96,7 +96,7 @@ Mpnn::Mpnn(Ctx& c, int nf, int layers, uint64_t seed) : c_(c) {
     grad_.alloc(sizeof(float) * P);
     m1_.alloc(sizeof(float) * P);
     m2_.alloc(sizeof(float) * P);
-    partials_.alloc(nn_partials_bytes());
+    partials_.alloc(nn_partials_bytes(sh_));
     launch_fill(c_, P, m1_.p, Prec::F32, 0.0);
     launch_fill(c_, P, m2_.p, Prec::F32, 0.0);
     set_params(p.data());
@@ -123,17 +123,15 @@ void Mpnn::reserve(int n) {
     x0_.alloc(sizeof(float) * n * sh_.din());
     h_.alloc(sizeof(float) * (L + 1) * n * H);
     m_.alloc(sizeof(float) * L * n * H);
-    dh_.alloc(sizeof(float) * n * H);
-    dh2_.alloc(sizeof(float) * n * H);
-    t_.alloc(sizeof(float) * n * H);
-    delta_.alloc(sizeof(double) * n * nf);
+    dh_.alloc(sizeof(float) * (L + 1) * n * H);
     diff_.alloc(sizeof(double) * n * nf);
     Adiff_.alloc(sizeof(double) * n * nf);
-    g_.alloc(sizeof(double) * n * nf);
     cap_ = n;
 }
 
-void Mpnn::forward(const NnGraph& g, const double* r1, double* delta, bool bf16) {
+void Mpnn::forward(const NnGraph& g, const double* r1, double* delta, bool bf16) { forward(g, r1, nullptr, delta, bf16); }
+
+void Mpnn::forward(const NnGraph& g, const double* r1, const double* e1, double* out, bool bf16) {
     FH_CHECK(g.nf == sh_.nf, -2, "network and operator have different face block sizes");
     FH_CHECK(g.n <= cap_, -2, "network workspace too small: reserve() first");
     const int n = g.n, nf = g.nf, L = sh_.layers;
@@ -141,85 +139,53 @@ void Mpnn::forward(const NnGraph& g, const double* r1, double* delta, bool bf16)
     const size_t es = bf16 ? 2 : 4;
     const char* P = (const char*)(bf16 ? p16_.p : p32_.p);
     auto par = [&](int64_t off) { return (const void*)(P + off * es); };
-    nn_prep(c_, n, nf, r1, g.invD32.as<float>(), v_.as<float>());
-    const void* xs[1] = {v_.p};
-    const void* ys[1] = {v_.p};
-    int sl[1] = {kNnSlotVV};
-    launch_dots(c_, (int64_t)n * nf, Prec::F32, 1, xs, ys, sl);
-    nn_input(c_, n, nf, v_.as<float>(), g.feat.as<float>(), kNnSlotVV, kNnSlotSigma, u_.as<float>(),
-             x0_.as<float>());
+    nn_prep(c_, n, nf, r1, g.invD32.as<float>(), v_.as<float>(), partials_.as<double>());
     float* h = h_.as<float>();
-    nn_encode(c_, n, sh_.din(), x0_.as<float>(), par(sh_.We()), par(sh_.be()), bf16, h);
+    nn_encode(c_, n, nf, partials_.as<double>(), v_.as<float>(), g.feat.as<float>(), kNnSlotSigma, par(sh_.We()),
+              par(sh_.be()), bf16, u_.as<float>(), bf16 ? nullptr : x0_.as<float>(), h);
     for (int l = 0; l < L; l++)
         nn_layer(c_, n, g.A->rowptr.as<int>(), g.A->colidx.as<int>(), g.w.as<float>(), h + l * nH, par(sh_.S(l)),
                  par(sh_.N(l)), par(sh_.c(l)), bf16, h + (l + 1) * nH, bf16 ? nullptr : m_.as<float>() + l * nH);
-    nn_out(c_, n, nf, h + L * nH, u_.as<float>(), par(sh_.Wo()), par(sh_.bo()), bf16, kNnSlotSigma, delta);
+    nn_out(c_, n, nf, h + L * nH, u_.as<float>(), par(sh_.Wo()), par(sh_.bo()), bf16, kNnSlotSigma, e1, out);
 }
 
-// After forward(train) into delta_: loss = (e1-delta)^T A (e1-delta) / e1^T r1
-// and g_ = dloss/ddelta = -2 A (e1 - delta) / (e1^T r1).
-double Mpnn::loss_and_seed(const NnGraph& g, const double* e1) {
-    const int64_t N = (int64_t)g.n * g.nf;
-    FH_HIP(hipMemcpyAsync(diff_.p, e1, sizeof(double) * N, hipMemcpyDeviceToDevice, c_.stream));
-    launch_axpby(c_, N, Prec::F64, delta_.p, diff_.p, -1.0, -1, -1, 1.0, -1, -1);
-    launch_bcsr(c_, *g.A, OP_SPMV, Prec::F64, diff_.p, nullptr, Adiff_.p, 1.0, 0.0, 0.0, nullptr, Prec::F64, nullptr,
-                0);
-    const void* xs[1] = {diff_.p};
-    const void* ys[1] = {Adiff_.p};
-    int sl[1] = {kNnSlotE};
-    launch_dots(c_, N, Prec::F64, 1, xs, ys, sl);
-    FH_HIP(hipMemcpyAsync(c_.h_scalars + kNnSlotE, c_.d_scalars + kNnSlotE, sizeof(double) * 2, hipMemcpyDeviceToHost,
-                          c_.stream));
-    c_.sync();
-    const double E = c_.h_scalars[kNnSlotE], E0 = c_.h_scalars[kNnSlotE0];
-    FH_CHECK(E0 > 0, -2, "training pair with zero energy (e1^T r1 <= 0)");
-    FH_HIP(hipMemcpyAsync(g_.p, Adiff_.p, sizeof(double) * N, hipMemcpyDeviceToDevice, c_.stream));
-    launch_axpby(c_, N, Prec::F64, Adiff_.p, g_.p, -2.0 / E0, -1, -1, 0.0, -1, -1);
-    return E / E0;
-}
-
-void Mpnn::backward(const NnGraph& g, const double* gdelta) {
-    const int n = g.n, nf = g.nf, L = sh_.layers, din = sh_.din();
-    const int64_t H = kNnHidden, nH = (int64_t)n * H;
+// Gradients of loss = (e1 - delta)^T A (e1 - delta) / e1^T r1 with respect to
+// all parameters, from Adiff_ = A (e1 - delta) and the device scalar e1^T r1
+// (dloss/ddelta = -2 A (e1 - delta) / (e1^T r1)).
+void Mpnn::backward(const NnGraph& g) {
+    const int n = g.n, L = sh_.layers;
+    const int64_t nH = (int64_t)n * kNnHidden;
     const float* P = p32_.as<float>();
-    float* G = grad_.as<float>();
-    double* part = partials_.as<double>();
     const float* h = h_.as<float>();
-    const float* m = m_.as<float>();
     float* dh = dh_.as<float>();
-    float* dh2 = dh2_.as<float>();
-    nn_out_back(c_, n, nf, gdelta, kNnSlotSigma, P + sh_.Wo(), gy_.as<float>(), dh);
-    nn_outer(c_, n, nf, (int)H, gy_.as<float>(), h + L * nH, part, G + sh_.Wo());
-    nn_outer(c_, n, nf, 1, gy_.as<float>(), nullptr, part, G + sh_.bo());
-    for (int l = L - 1; l >= 0; l--) {
-        nn_relu_back(c_, nH, h + (l + 1) * nH, dh);
-        nn_outer(c_, n, (int)H, (int)H, dh, h + l * nH, part, G + sh_.S(l));
-        nn_outer(c_, n, (int)H, (int)H, dh, m + l * nH, part, G + sh_.N(l));
-        nn_outer(c_, n, (int)H, 1, dh, nullptr, part, G + sh_.c(l));
-        nn_back_self(c_, n, dh, P + sh_.S(l), P + sh_.N(l), dh2, t_.as<float>());
-        nn_back_gather(c_, n, g.A->rowptr.as<int>(), g.A->colidx.as<int>(), g.wT.as<float>(), t_.as<float>(), dh2);
-        std::swap(dh, dh2);
-    }
-    nn_relu_back(c_, nH, h, dh);
-    nn_outer(c_, n, (int)H, din, dh, x0_.as<float>(), part, G + sh_.We());
-    nn_outer(c_, n, (int)H, 1, dh, nullptr, part, G + sh_.be());
+    nn_out_back(c_, n, g.nf, Adiff_.as<double>(), kNnSlotE0, kNnSlotSigma, P + sh_.Wo(), h + L * nH, gy_.as<float>(),
+                dh + L * nH);
+    for (int l = L - 1; l >= 0; l--)
+        nn_layer_back(c_, n, g.A->rowptr.as<int>(), g.A->colidx.as<int>(), g.wT.as<float>(), dh + (l + 1) * nH,
+                      P + sh_.S(l), P + sh_.N(l), h + l * nH, dh + l * nH);
+    nn_weight_grads(c_, n, sh_, gy_.as<float>(), dh, h, m_.as<float>(), x0_.as<float>(), partials_.as<double>(),
+                    grad_.as<float>());
 }
 
 double Mpnn::loss_grad(const NnGraph& g, const double* r1, const double* e1, float* grad_host) {
     reserve(g.n);
     const int64_t N = (int64_t)g.n * g.nf;
-    const void* xs[1] = {e1};
-    const void* ys[1] = {r1};
-    int sl[1] = {kNnSlotE0};
-    launch_dots(c_, N, Prec::F64, 1, xs, ys, sl);
-    forward(g, r1, delta_.as<double>(), false);
-    const double loss = loss_and_seed(g, e1);
-    backward(g, g_.as<double>());
-    if (grad_host) {
+    forward(g, r1, e1, diff_.as<double>(), false);
+    launch_bcsr(c_, *g.A, OP_SPMV, Prec::F64, diff_.p, nullptr, Adiff_.p, 1.0, 0.0, 0.0, nullptr, Prec::F64, nullptr,
+                0);
+    const void* xs[2] = {diff_.p, e1};
+    const void* ys[2] = {Adiff_.p, r1};
+    int sl[2] = {kNnSlotE, kNnSlotE0};
+    launch_dots(c_, N, Prec::F64, 2, xs, ys, sl);
+    FH_HIP(hipMemcpyAsync(c_.h_scalars + kNnSlotE, c_.d_scalars + kNnSlotE, sizeof(double) * 2, hipMemcpyDeviceToHost,
+                          c_.stream));
+    backward(g);
+    if (grad_host)
         FH_HIP(hipMemcpyAsync(grad_host, grad_.p, sizeof(float) * sh_.total(), hipMemcpyDeviceToHost, c_.stream));
-        c_.sync();
-    }
-    return loss;
+    c_.sync();
+    const double E = c_.h_scalars[kNnSlotE], E0 = c_.h_scalars[kNnSlotE0];
+    FH_CHECK(E0 > 0, -2, "training pair with zero energy (e1^T r1 <= 0)");
+    return E / E0;
 }
 
 double Mpnn::train_step(const NnGraph& g, const double* r1, const double* e1, float lr) {

@@ -29,7 +29,7 @@ namespace fh {
 constexpr int kNnHidden = 32;
 constexpr int kNnMaxLayers = 6;
 // device scalar slots used by the network
-constexpr int kNnSlotVV = 480, kNnSlotSigma = 481, kNnSlotS1 = 482, kNnSlotS2 = 483, kNnSlotE = 484,
+constexpr int kNnSlotSigma = 481, kNnSlotS1 = 482, kNnSlotS2 = 483, kNnSlotE = 484,
               kNnSlotE0 = 485;
 
 struct NnShape {
@@ -80,26 +80,32 @@ private:
     DevBuf p32_, p16_, grad_, m1_, m2_, partials_;
     int step_ = 0;
     int cap_ = 0;
-    DevBuf v_, u_, x0_, gy_, h_, m_, dh_, dh2_, t_, delta_, diff_, Adiff_, g_;
-    void backward(const NnGraph& g, const double* gdelta);
-    double loss_and_seed(const NnGraph& g, const double* e1);
+    DevBuf v_, u_, x0_, gy_, h_, m_, dh_, diff_, Adiff_;
+    // delta into out, or e1 - delta when e1 is not null
+    void forward(const NnGraph& g, const double* r1, const double* e1, double* out, bool bf16);
+    void backward(const NnGraph& g);
 };
 
 // ------------------------------------------------------------ launchers
-void nn_prep(Ctx& c, int n, int nf, const double* r1, const float* invD, float* v);
-void nn_input(Ctx& c, int n, int nf, const float* v, const float* feat, int slot_vv, int slot_sigma, float* u,
-              float* x0);
-void nn_encode(Ctx& c, int n, int din, const float* x, const void* We, const void* be, bool bf16, float* h);
+// v = D^-1 r1 and partial sums of |v|^2, which nn_encode adds.
+void nn_prep(Ctx& c, int n, int nf, const double* r1, const float* invD, float* v, double* partials);
+void nn_encode(Ctx& c, int n, int nf, const double* partials, const float* v, const float* feat, int slot_sigma,
+               const void* We, const void* be, bool bf16, float* u, float* x0, float* h);
 void nn_layer(Ctx& c, int n, const int* rp, const int* ci, const float* w, const float* hin, const void* S,
               const void* N, const void* cb, bool bf16, float* hout, float* m_out);
+// Gradient at a layer's input h from that at its output (after the relu).
+void nn_layer_back(Ctx& c, int n, const int* rp, const int* ci, const float* wT, const float* dpre, const float* S,
+                   const float* N, const float* h, float* dprev);
+// delta, or e1 - delta when e1 is not null.
 void nn_out(Ctx& c, int n, int nf, const float* h, const float* u, const void* Wo, const void* bo, bool bf16,
-            int slot_sigma, double* delta);
-void nn_out_back(Ctx& c, int n, int nf, const double* g, int slot_sigma, const float* Wo, float* gy, float* dh);
-void nn_relu_back(Ctx& c, int64_t count, const float* h, float* dh);
-void nn_back_self(Ctx& c, int n, const float* dpre, const float* S, const float* N, float* dprev, float* tvec);
-void nn_back_gather(Ctx& c, int n, const int* rp, const int* ci, const float* wT, const float* tvec, float* dprev);
-void nn_outer(Ctx& c, int n, int da, int db, const float* A, const float* B, double* partials, float* grad);
-size_t nn_partials_bytes();
+            int slot_sigma, const double* e1, double* delta);
+void nn_out_back(Ctx& c, int n, int nf, const double* Adiff, int slot_e0, int slot_sigma, const float* Wo,
+                 const float* h, float* gy, float* dh);
+// Gradients of all parameters; dh: the gradients at the outputs of the encoder
+// and the layers (n x 32 each), h their outputs, m the layers' aggregates.
+void nn_weight_grads(Ctx& c, int n, const NnShape& sh, const float* gy, const float* dh, const float* h,
+                     const float* m, const float* x0, double* partials, float* grad);
+size_t nn_partials_bytes(const NnShape& sh);
 void nn_adam(Ctx& c, int np, float* w, const float* g, float* m1, float* m2, float lr, float b1, float b2, float eps,
              int step, void* wb);
 void nn_to_bf16(Ctx& c, int np, const float* w, void* wb);

@@ -2,17 +2,19 @@
 // the face graph of the condensed operator (one node per block row, edges =
 // off-diagonal blocks), hidden width 32.
 //
-// Layout: node features are row-major n x 32 FP32 arrays (one 128-byte row
-// per face), so the 32 lanes of a node read or write one row with one
-// coalesced access.  A workgroup of 256 threads = 8 nodes x 32 channels; every
-// lane computes one output channel.  The message-passing layer keeps its
-// lane's weight rows in registers and strides over node batches staged in
-// LDS; the smaller kernels read the weights from the cache.  Weights are FP32
-// for training and BF16 (FP32 accumulate) for inference.
+// Layout: node features are row-major n x 32 FP32 arrays, one 128-byte row per
+// face.  The message-passing layer (forward, inference and backward) gathers
+// neighbour rows with 8 lanes of 16 bytes each and multiplies on the matrix
+// cores: FP32 for training, BF16 operands (FP32 sums) for inference.  Weights
+// are FP32 for training and BF16 for inference.
 //
-// Weight gradients are sums over nodes of outer products; each workgroup of
-// a fixed-size grid accumulates its own share in FP64 and a second kernel
-// adds the shares in a fixed order, so gradients are deterministic.
+// Weight gradients are sums over nodes of outer products, formed for all
+// layers in one launch on v_mfma_f64_16x16x4f64: FP64 sums per workgroup of a
+// fixed-size grid, added in a fixed order by a second kernel, so gradients are
+// deterministic.
+#include <algorithm>
+
+#include "fh_lane.h"
 #include "fh_nn.h"
 
 namespace fh {
@@ -20,7 +22,9 @@ namespace {
 
 constexpr int H = kNnHidden;  // 32
 constexpr int kNodesPerWG = 8;
-constexpr int kOuterWGs = 256;
+constexpr int kOuterWGs = 128;
+constexpr int kMaxDin = 12, kMaxNf = 10;
+constexpr int kPrepWGs = 1024;  // partial sums of |v|^2
 
 struct bf16w {
     uint16_t u;
@@ -28,217 +32,119 @@ struct bf16w {
 __device__ __forceinline__ float wload(const float* p) { return *p; }
 __device__ __forceinline__ float wload(const bf16w* p) { return __uint_as_float(((uint32_t)p->u) << 16); }
 
-// v = D^-1 r1 (FP32), thread per unknown.
-__global__ void k_nn_prep(int n, int nf, const double* __restrict__ r1, const float* __restrict__ invD,
-                          float* __restrict__ v) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)n * nf) return;
-    const int i = (int)(t / nf), a = (int)(t - (int64_t)i * nf);
-    const float* D = invD + ((int64_t)i * nf + a) * nf;
-    const double* r = r1 + (int64_t)i * nf;
-    float s = 0.f;
-    for (int b = 0; b < nf; b++) s += D[b] * (float)r[b];
-    v[t] = s;
+// v = D^-1 r1 (FP32) and the workgroup's share of |v|^2 (FP64), 256 / nf block
+// rows at a time: their inverse blocks (one contiguous span) and entries of r1
+// go through LDS, then thread t forms entry t of the tile.  Bound by reading
+// the inverse blocks; a thread per unknown that reads its row of D strided
+// took 21.5 us for 95 232 blocks of 10 x 10 (38 MB).
+__global__ __launch_bounds__(256) void k_nn_prep(int n, int nf, const double* __restrict__ r1,
+                                                 const float* __restrict__ invD, float* __restrict__ v,
+                                                 double* __restrict__ partials) {
+    __shared__ float sD[256 * kMaxNf], sr[256];
+    __shared__ double sw[4];
+    const int t = threadIdx.x, R = 256 / nf, b = t / nf;
+    double vv = 0;
+    for (int64_t r0 = (int64_t)blockIdx.x * R; r0 < n; r0 += (int64_t)gridDim.x * R) {
+        const int rows = (int)min((int64_t)R, n - r0), nv = rows * nf, ne = nv * nf;
+        const float* D = invD + r0 * nf * nf;
+        for (int e = t; e < ne; e += 256) sD[e] = __builtin_nontemporal_load(D + e);
+        if (t < nv) sr[t] = (float)r1[r0 * nf + t];
+        __syncthreads();
+        if (t < nv) {
+            float s = 0.f;
+            for (int j = 0; j < nf; j++) s += sD[t * nf + j] * sr[b * nf + j];
+            v[r0 * nf + t] = s;
+            vv += (double)s * (double)s;
+        }
+        __syncthreads();
+    }
+    for (int o = 32; o > 0; o >>= 1) vv += __shfl_down(vv, o, 64);
+    if ((t & 63) == 0) sw[t >> 6] = vv;
+    __syncthreads();
+    if (t == 0) partials[blockIdx.x] = ((sw[0] + sw[1]) + sw[2]) + sw[3];
 }
 
-// sigma = sqrt(<v,v> / (n nf)); u = v / sigma; x0 = [u, feat]; sigma -> s[slot_sigma].
-__global__ void k_nn_input(int n, int nf, const float* __restrict__ v, const float* __restrict__ feat,
-                           double* s, int slot_vv, int slot_sigma, float* __restrict__ u, float* __restrict__ x0) {
-    const int din = nf + 2;
-    const double sig = sqrt(s[slot_vv] / ((double)n * nf));
-    const float inv = sig > 0 ? (float)(1.0 / sig) : 0.f;
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) s[slot_sigma] = sig;
-    if (t >= (int64_t)n * din) return;
-    const int i = (int)(t / din), a = (int)(t - (int64_t)i * din);
-    float val;
-    if (a < nf) {
-        val = v[(int64_t)i * nf + a] * inv;
-        u[(int64_t)i * nf + a] = val;
-    } else
-        val = feat[(int64_t)i * 2 + (a - nf)];
-    x0[t] = val;
-}
-
-// Encoder: h = relu(We x + be), x of width din <= kMaxDin.  Lane c keeps row c
-// of We in registers; the grid strides over nodes.
-constexpr int kMaxDin = 12;
-constexpr int kEncodeMaxWGs = 8192;
+// Encoder: sigma = sqrt(<v, v> / (n nf)) from the npart partial sums (added by
+// every workgroup in the same order; the first one writes sigma to
+// s[slot_sigma]), u = v / sigma, x = [u, feat] (stored when x0 is not null)
+// and h = relu(We x + be).  Lane c keeps row c of We in registers; the inputs
+// of 64 nodes at a time are staged in LDS.
+constexpr int kEncodeNodes = 64, kEncodeMaxWGs = 1536;
 
 template <class TW>
-__global__ __launch_bounds__(256) void k_nn_encode(int n, int din, const float* __restrict__ x,
-                                                    const TW* __restrict__ We, const TW* __restrict__ be,
-                                                    float* __restrict__ h) {
+__global__ __launch_bounds__(256) void k_nn_encode(int n, int nf, int npart, const double* __restrict__ partials,
+                                                    const float* __restrict__ v, const float* __restrict__ feat,
+                                                    double* s, int slot_sigma, const TW* __restrict__ We,
+                                                    const TW* __restrict__ be, float* __restrict__ u,
+                                                    float* __restrict__ x0, float* __restrict__ h) {
+    __shared__ float sx[kEncodeNodes * kMaxDin];
     __shared__ float sWe[H * kMaxDin + H];
-    for (int e = threadIdx.x; e < H * din; e += blockDim.x) sWe[e] = wload(We + e);
-    if (threadIdx.x < H) sWe[H * kMaxDin + threadIdx.x] = wload(be + threadIdx.x);
+    __shared__ double sw[4];
+    const int t = threadIdx.x, din = nf + 2;
+    double vv = 0;
+    for (int i = t; i < npart; i += 256) vv += partials[i];
+    for (int o = 32; o > 0; o >>= 1) vv += __shfl_down(vv, o, 64);
+    if ((t & 63) == 0) sw[t >> 6] = vv;
+    for (int e = t; e < H * din; e += 256) sWe[e] = wload(We + e);
+    if (t < H) sWe[H * kMaxDin + t] = wload(be + t);
     __syncthreads();
-    const int c = threadIdx.x & (H - 1);
+    const double sig = sqrt((((sw[0] + sw[1]) + sw[2]) + sw[3]) / ((double)n * nf));
+    const float inv = sig > 0 ? (float)(1.0 / sig) : 0.f;
+    if (blockIdx.x == 0 && t == 0) s[slot_sigma] = sig;
+    const int c = t & (H - 1), q = t >> 5;
     float wr[kMaxDin];
 #pragma unroll
     for (int k = 0; k < kMaxDin; k++) wr[k] = k < din ? sWe[c * din + k] : 0.f;
     const float bias = sWe[H * kMaxDin + c];
-    for (int64_t i = (int64_t)blockIdx.x * kNodesPerWG + (threadIdx.x >> 5); i < n;
-         i += (int64_t)gridDim.x * kNodesPerWG) {
-        float acc = bias;
-        const float* xi = x + i * din;
-#pragma unroll
-        for (int k = 0; k < kMaxDin; k++)
-            if (k < din) acc += wr[k] * xi[k];
-        h[i * H + c] = acc > 0.f ? acc : 0.f;
-    }
-}
-
-// Message-passing layer: m_i = sum_j w_ij h_j ; h'_i = relu(S h_i + N m_i + c).
-// m is stored for the backward pass when m_out != nullptr.
-//
-// Lane c of a 32-lane half-wave owns output channel c and keeps row c of S
-// and of N in registers for the whole launch (staged once per workgroup, not
-// once per node).  The grid strides over batches of kLayerBatch nodes: every
-// thread gathers kLayerBatch / 8 nodes' (h_i, m_i) rows into LDS, then
-// computes their channel c from LDS broadcasts (16-byte reads; the row pitch
-// of 2H + 4 floats puts the two half-waves' rows in different banks).  The
-// batch loop bound depends on blockIdx only, so both barriers are uniform.
-constexpr int kLayerBatch = 32;            // nodes per workgroup iteration
-constexpr int kLayerPer = kLayerBatch / 8; // nodes per thread per iteration
-constexpr int kLayerPitch = 2 * H + 4;
-constexpr int kLayerMaxWGs = 768;  // 3 workgroups of 4 waves per CU (164 VGPRs: 3 waves per SIMD)
-
-template <class TW>
-__global__ __launch_bounds__(256) void k_nn_layer(int n, const int* __restrict__ rp, const int* __restrict__ ci,
-                                                   const float* __restrict__ w, const float* __restrict__ hin,
-                                                   const TW* __restrict__ S, const TW* __restrict__ N,
-                                                   const TW* __restrict__ cb, float* __restrict__ hout,
-                                                   float* __restrict__ m_out) {
-    __shared__ __align__(16) float sx[kLayerBatch][kLayerPitch];
-    __shared__ float sW[2 * H * H];  // S^T then N^T: sW[k H + c] = S[c][k]
-    // Weights reach the registers through LDS: one coalesced read per
-    // workgroup (every lane of the grid reading the same few lines from L2
-    // would serialise on their channels).
-    for (int e = threadIdx.x; e < H * H; e += blockDim.x) {
-        const int row = e / H, k = e - row * H;
-        sW[k * H + row] = wload(S + e);
-        sW[H * H + k * H + row] = wload(N + e);
-    }
-    __syncthreads();
-    const int c = threadIdx.x & (H - 1), q = threadIdx.x >> 5;
-    float ws[H], wn[H];
-#pragma unroll
-    for (int k = 0; k < H; k++) {
-        ws[k] = sW[k * H + c];
-        wn[k] = sW[H * H + k * H + c];
-    }
-    const float bias = wload(cb + c);
-    for (int64_t base = (int64_t)blockIdx.x * kLayerBatch; base < n; base += (int64_t)gridDim.x * kLayerBatch) {
-        // gather.  Lane c of the half-wave fetches edge c of each of its
-        // kLayerPer rows (one coalesced load for the row's columns and
-        // weights); edge e is then broadcast from lane e, and the neighbour
-        // rows of four edge positions x kLayerPer nodes are loaded before
-        // they are summed (edge order kept per node).  Rows longer than 32
-        // edges read the rest directly.
-        int beg[kLayerPer], deg[kLayerPer], dmax = 0;
-        float m[kLayerPer], hs[kLayerPer];
-#pragma unroll
-        for (int r = 0; r < kLayerPer; r++) {
-            const int64_t i = base + r * 8 + q;
-            beg[r] = 0;
-            deg[r] = 0;
-            hs[r] = 0.f;
-            m[r] = 0.f;
-            if (i < n) {
-                beg[r] = rp[i];
-                deg[r] = rp[i + 1] - beg[r];
-                hs[r] = hin[i * H + c];
-            }
-            dmax = deg[r] > dmax ? deg[r] : dmax;
+    for (int64_t i0 = (int64_t)blockIdx.x * kEncodeNodes; i0 < n; i0 += (int64_t)gridDim.x * kEncodeNodes) {
+        const int nn = (int)min((int64_t)kEncodeNodes, n - i0);
+        for (int e = t; e < nn * nf; e += 256) {
+            const int i = e / nf, a = e - i * nf;
+            const float val = v[i0 * nf + e] * inv;
+            u[i0 * nf + e] = val;
+            sx[i * kMaxDin + a] = val;
         }
-        dmax = max(dmax, __shfl_xor(dmax, 32));  // wave-uniform trip count
-        int colv[kLayerPer];
-        float wv[kLayerPer];
-#pragma unroll
-        for (int r = 0; r < kLayerPer; r++) {
-            colv[r] = c < deg[r] ? ci[beg[r] + c] : 0;
-            wv[r] = c < deg[r] ? w[beg[r] + c] : 0.f;
-        }
-        for (int e0 = 0; e0 < dmax; e0 += 4) {
-            float v[4][kLayerPer], wt[4][kLayerPer];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int e = e0 + u;
-#pragma unroll
-                for (int r = 0; r < kLayerPer; r++) {
-                    int col;
-                    float we;
-                    if (e < 32) {
-                        col = __shfl(colv[r], e, 32);
-                        we = __shfl(wv[r], e, 32);
-                    } else {
-                        col = e < deg[r] ? ci[beg[r] + e] : 0;
-                        we = e < deg[r] ? w[beg[r] + e] : 0.f;
-                    }
-                    wt[u][r] = we;
-                    v[u][r] = e < deg[r] ? hin[(int64_t)col * H + c] : 0.f;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int r = 0; r < kLayerPer; r++)
-                    if (e0 + u < deg[r]) m[r] += wt[u][r] * v[u][r];
-        }
-#pragma unroll
-        for (int r = 0; r < kLayerPer; r++) {
-            const int slot = r * 8 + q;
-            const int64_t i = base + slot;
-            if (m_out && i < n) m_out[i * H + c] = m[r];
-            sx[slot][c] = hs[r];
-            sx[slot][H + c] = m[r];
-        }
+        for (int e = t; e < nn * 2; e += 256) sx[(e >> 1) * kMaxDin + nf + (e & 1)] = feat[i0 * 2 + e];
         __syncthreads();
-#pragma unroll
-        for (int r = 0; r < kLayerPer; r++) {
-            const int slot = r * 8 + q;
-            const int64_t i = base + slot;
-            const float4* x4 = reinterpret_cast<const float4*>(&sx[slot][0]);
+        if (x0)
+            for (int e = t; e < nn * din; e += 256) x0[i0 * din + e] = sx[e / din * kMaxDin + e % din];
+        for (int i = q; i < nn; i += kNodesPerWG) {
             float acc = bias;
 #pragma unroll
-            for (int k4 = 0; k4 < H / 4; k4++) {
-                const float4 hv = x4[k4], mv = x4[H / 4 + k4];
-                acc += ws[4 * k4 + 0] * hv.x + wn[4 * k4 + 0] * mv.x;
-                acc += ws[4 * k4 + 1] * hv.y + wn[4 * k4 + 1] * mv.y;
-                acc += ws[4 * k4 + 2] * hv.z + wn[4 * k4 + 2] * mv.z;
-                acc += ws[4 * k4 + 3] * hv.w + wn[4 * k4 + 3] * mv.w;
-            }
-            if (i < n) hout[i * H + c] = acc > 0.f ? acc : 0.f;
+            for (int k = 0; k < kMaxDin; k++)
+                if (k < din) acc += wr[k] * sx[i * kMaxDin + k];
+            h[(i0 + i) * H + c] = acc > 0.f ? acc : 0.f;
         }
         __syncthreads();
     }
 }
 
-// Inference layer (BF16 weights): the same layer with the dense part on the
-// matrix cores.  A wave owns tiles of 32 consecutive nodes.
-//  1. The tile's row pointers come in one load, its edge list (contiguous in
-//     the CSR arrays) in a few coalesced loads, into the wave's LDS.
-//  2. Each half-wave walks the edges of its 16 nodes in order, kMChunk rows
-//     in flight (lane c = channel c), keeps a running sum per node and writes
-//     (h_i, m_i) to the tile in LDS as BF16.  Tiles with more than kMEdges
-//     edges walk their nodes one by one instead.
-//  3. Four v_mfma_f32_32x32x16_bf16 multiply the 32 x 64 tile by the 64 x 32
-//     matrix [S N]^T (FP32 accumulate).  A lane supplies row lane%32 of the
-//     tile and column lane%32 of the weights with the same k elements, and
-//     receives column lane%32 of the product: rows 8 (r / 4) + 4 (lane / 32)
-//     + r % 4 of its 16 accumulators.
-// Activations are rounded to BF16 (round to nearest even) for the product;
-// the neighbour sum m_i is accumulated in FP32 in edge order.
+// Message-passing layer of 16 nodes per wavefront:
+//   m_i = sum_j w_ij h_j (edge order, FP32);  y_i = S h_i + N m_i + c
+//   LAYER_TRAIN  out = relu(y), m stored for the backward pass (FP32 products)
+//   LAYER_INFER  out = relu(y), h and m rounded to BF16 for the products
+//   LAYER_BACK   h, w, c: the gradient at the layer's output, the weights of
+//                the reverse edges, none; S and N transposed; out = y where
+//                the layer's input (mask) is positive, else 0: the gradient at
+//                the previous layer's output.  (N^T m with m gathered first is
+//                the sum of the neighbours' N^T h.)
+// 8 lanes of 16 bytes read a 128-byte row, so one load instruction fetches 8
+// neighbour rows; the lane group g sums the edges of nodes g and g + 8, their
+// next kGather rows each in flight together (column indexes and weights of 8
+// edges come in one load and are passed on by shuffles).  The 16 x 64 operand
+// [h m] goes through LDS to the matrix cores: v_mfma_f32_16x16x4f32 or
+// v_mfma_f32_16x16x32_bf16, lane l supplying row (column) l % 16 and receiving
+// rows 4 (l / 16) + v of column l % 16.  Bound by the latency of the gather:
+// 16 nodes instead of 32 per wavefront and 16-byte lanes halve the number of
+// dependent loads (95 232 nodes, 1.02 M edges, BF16: 13.4 us; 36.5 us with 4-byte
+// lanes and 32 nodes).  Workgroups of one XCD take a contiguous range of nodes, whose
+// neighbour rows its L2 then holds.
+enum { LAYER_TRAIN = 0, LAYER_INFER = 1, LAYER_BACK = 2 };
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-constexpr int kMTile = 32;
-constexpr int kMWaves = 4;
-constexpr int kMBatch = kMTile * kMWaves;  // nodes per workgroup iteration
-constexpr int kMPitch = 2 * H + 8;         // BF16 elements per tile row (144 bytes)
-constexpr int kMEdges = 384;               // staged edges per tile
-constexpr int kMChunk = 16;                // neighbour rows in flight per half-wave
-constexpr int kMMaxWGs = 1024;             // 4 workgroups per CU
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+constexpr int kLTile = 16, kLWaves = 4;
+constexpr int kGather = 6;
 
 __device__ __forceinline__ __bf16 to_bf16(float f) {
     uint32_t u = __float_as_uint(f);
@@ -246,133 +152,162 @@ __device__ __forceinline__ __bf16 to_bf16(float f) {
     return __builtin_bit_cast(__bf16, (uint16_t)(u >> 16));
 }
 
-__global__ __launch_bounds__(256) void k_nn_layer_mfma(int n, const int* __restrict__ rp, const int* __restrict__ ci,
-                                                        const float* __restrict__ w, const float* __restrict__ hin,
-                                                        const bf16w* __restrict__ S, const bf16w* __restrict__ N,
-                                                        const bf16w* __restrict__ cb, float* __restrict__ hout) {
-    __shared__ __align__(16) __bf16 tile[kMWaves][kMTile][kMPitch];
-    __shared__ uint16_t sB[2 * H * H];  // sB[k H + j] = [S N]^T[k][j]
-    __shared__ int s_col[kMWaves][kMEdges];
-    __shared__ float s_w[kMWaves][kMEdges];
-    __shared__ uint8_t s_node[kMWaves][kMEdges];
-    __shared__ int s_row[kMWaves][kMTile + 1];
-    for (int e = threadIdx.x; e < H * H; e += blockDim.x) {
-        const int row = e / H, k = e - row * H;
-        sB[k * H + row] = S[e].u;
-        sB[(H + k) * H + row] = N[e].u;
+template <int MODE>
+__global__ __launch_bounds__(kLWaves * 64) void k_nn_layer(int n, const int* __restrict__ rp,
+                                                            const int* __restrict__ ci, const float* __restrict__ w,
+                                                            const float* __restrict__ hin, const void* Sv,
+                                                            const void* Nv, const void* cv,
+                                                            const float* __restrict__ mask, float* __restrict__ hout,
+                                                            float* __restrict__ m_out) {
+    constexpr bool BF = MODE == LAYER_INFER, BACK = MODE == LAYER_BACK;
+    using TW = std::conditional_t<BF, bf16w, float>;
+    using TT = std::conditional_t<BF, __bf16, float>;
+    constexpr int PITCH = BF ? 2 * H + 8 : 2 * H + 4;  // rows 16 bytes apart in their banks
+    __shared__ __align__(16) TT tiles[kLWaves][kLTile * PITCH];
+    const TW *S = (const TW*)Sv, *N = (const TW*)Nv;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int wg = blockIdx.x;
+    {
+        const int nwg = gridDim.x, xcd = wg & 7, per = nwg >> 3, rem = nwg & 7;
+        wg = xcd * per + (xcd < rem ? xcd : rem) + (wg >> 3);
     }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, half = lane >> 5, c = lane & 31;
-    bf16x8_t bop[4];
+    const int64_t i0 = ((int64_t)wg * kLWaves + wave) * kLTile;
+    if (i0 >= n) return;  // wavefront-uniform; no barrier follows
+    const int nt = (int)min((int64_t)kLTile, n - i0);
+    TT* tl = tiles[wave];
+    // edges: lane group g (8 lanes) sums nodes g and g + 8
+    const int g = lane >> 3, c4 = lane & 7, gl = lane & 56;
+    const int rpv = rp[i0 + min(lane, nt)];
+    int beg[2], deg[2];
 #pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int u = 0; u < 8; u++) bop[t][u] = __builtin_bit_cast(__bf16, sB[(16 * t + 8 * half + u) * H + c]);
-    const float bias = wload(cb + c);
-    // XCD-aware batch order: workgroups are dealt to the 8 XCDs round robin,
-    // so XCD x (blockIdx % 8) walks the x-th contiguous slab of batches and
-    // the neighbour rows a tile gathers were mostly fetched into the same
-    // XCD's L2 by the tiles next to it.
-    const int64_t nbat = ((int64_t)n + kMBatch - 1) / kMBatch;
-    int64_t first = blockIdx.x, end = nbat, step = gridDim.x;
-    if (gridDim.x % 8 == 0) {
-        const int64_t slab = (nbat + 7) / 8, xcd = blockIdx.x % 8;
-        first = xcd * slab + blockIdx.x / 8;
-        end = min(nbat, (xcd + 1) * slab);
-        step = gridDim.x / 8;
+    for (int r = 0; r < 2; r++) {
+        const int k = g + 8 * r;
+        beg[r] = __shfl(rpv, min(k, nt), 64);
+        deg[r] = __shfl(rpv, min(k + 1, nt), 64) - beg[r];
     }
-    for (int64_t b = first; b < end; b += step) {
-        const int64_t tb = b * kMBatch + (int64_t)wv * kMTile;
-        const int nt = (int)max<int64_t>(0, min<int64_t>(kMTile, (int64_t)n - tb));  // nodes of this tile
-        // 1. row pointers and edge list
-        const int rpv = lane <= nt && nt > 0 ? rp[tb + lane] : 0;
-        const int e_base = __shfl(rpv, 0);
-        const int ne = __shfl(rpv, nt) - e_base;
-        const bool staged = ne <= kMEdges;
-        if (lane <= nt) s_row[wv][lane] = rpv - e_base;
-        if (staged) {
-            for (int e = lane; e < ne; e += 64) {
-                s_col[wv][e] = ci[e_base + e];
-                s_w[wv][e] = w[e_base + e];
-            }
-            const int rnext = __shfl(rpv, lane + 1 < 64 ? lane + 1 : 63);
-            if (lane < nt)
-                for (int e = rpv - e_base; e < rnext - e_base; e++) s_node[wv][e] = (uint8_t)lane;
+    floatx4 own[2], m[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int k = g + 8 * r;
+        own[r] = k < nt ? *(const floatx4*)(hin + (i0 + k) * H + 4 * c4) : floatx4{0.f, 0.f, 0.f, 0.f};
+        m[r] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    int dmax = max(deg[0], deg[1]);
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) dmax = max(dmax, __shfl_xor(dmax, o, 64));
+    int colv[2];
+    float wv[2];
+    auto load_edges = [&](int e0) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            const bool ok = c4 < kGather && e0 + c4 < deg[r];
+            colv[r] = ok ? ci[beg[r] + e0 + c4] : 0;
+            wv[r] = ok ? w[beg[r] + e0 + c4] : 0.f;
         }
-        __syncthreads();
-        // 2. (h_i, m_i) rows of the tile
-        const int r0 = min(16 * half, nt), r1 = min(16 * half + 16, nt);
-        {
-            float hs[16];
+    };
+    load_edges(0);
+    for (int e0 = 0; e0 < dmax; e0 += kGather) {
+        floatx4 x[2][kGather];
+        float we[2][kGather];
 #pragma unroll
-            for (int r = 0; r < 16; r++) hs[r] = r0 + r < r1 ? hin[(tb + r0 + r) * H + c] : 0.f;
+        for (int r = 0; r < 2; r++)
 #pragma unroll
-            for (int r = 0; r < 16; r++)
-                if (r0 + r < r1) {
-                    tile[wv][r0 + r][c] = to_bf16(hs[r]);
-                    tile[wv][r0 + r][H + c] = to_bf16(0.f);
-                }
-        }
-        if (staged) {
-            const int es = r0 < r1 ? s_row[wv][r0] : 0, ee = r0 < r1 ? s_row[wv][r1] : 0;
-            int cur = r0;
-            float run = 0.f;
-            for (int e0 = es; e0 < ee; e0 += kMChunk) {
-                float v[kMChunk];
-#pragma unroll
-                for (int u = 0; u < kMChunk; u++) {
-                    const int e = e0 + u;
-                    v[u] = e < ee ? hin[(int64_t)s_col[wv][e] * H + c] : 0.f;
-                }
-#pragma unroll
-                for (int u = 0; u < kMChunk; u++) {
-                    const int e = e0 + u;
-                    if (e < ee) {
-                        const int nd = s_node[wv][e];
-                        if (nd != cur) {
-                            tile[wv][cur][H + c] = to_bf16(run);
-                            run = 0.f;
-                            cur = nd;
-                        }
-                        run += s_w[wv][e] * v[u];
-                    }
-                }
+            for (int k = 0; k < kGather; k++) {
+                const int col = __shfl(colv[r], gl + k, 64);
+                we[r][k] = __shfl(wv[r], gl + k, 64);
+                if (e0 + k < deg[r]) x[r][k] = *(const floatx4*)(hin + (int64_t)col * H + 4 * c4);
             }
-            if (ee > es) tile[wv][cur][H + c] = to_bf16(run);
+        load_edges(e0 + kGather);
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int k = 0; k < kGather; k++)
+                if (e0 + k < deg[r]) {
+#pragma unroll
+                    for (int a = 0; a < 4; a++) m[r][a] += we[r][k] * x[r][k][a];
+                }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int k = g + 8 * r;
+        if (MODE == LAYER_TRAIN && k < nt) *(floatx4*)(m_out + (i0 + k) * H + 4 * c4) = m[r];
+        if constexpr (BF) {
+            bf16x4_t hb, mb;
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                hb[a] = to_bf16(own[r][a]);
+                mb[a] = to_bf16(m[r][a]);
+            }
+            *(bf16x4_t*)(tl + k * PITCH + 4 * c4) = hb;
+            *(bf16x4_t*)(tl + k * PITCH + H + 4 * c4) = mb;
         } else {
-            for (int r = r0; r < r1; r++) {
-                const int64_t i = tb + r;
-                float m = 0.f;
-                for (int p = rp[i]; p < rp[i + 1]; p++) m += w[p] * hin[(int64_t)ci[p] * H + c];
-                tile[wv][r][H + c] = to_bf16(m);
+            *(floatx4*)(tl + k * PITCH + 4 * c4) = own[r];
+            *(floatx4*)(tl + k * PITCH + H + 4 * c4) = m[r];
+        }
+    }
+    lds_order();
+    // [h m] (16 x 64) times [S N]^T (64 x 32); rows >= nt are zero
+    const int lr = lane >> 4, lc = lane & 15;
+    floatx4 acc[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const float b = BACK ? 0.f : wload((const TW*)cv + 16 * j + lc);
+        acc[j] = floatx4{b, b, b, b};
+    }
+    if constexpr (BF) {
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const bf16x8_t a = *(const bf16x8_t*)(tl + lc * PITCH + 32 * t + 8 * lr);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                // entries k = 8 lr .. 8 lr + 7 of row 16 j + lc of S (t = 0) or N
+                const bf16x8_t b = *(const bf16x8_t*)((t == 0 ? S : N) + (16 * j + lc) * H + 8 * lr);
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[j], 0, 0, 0);
             }
         }
-        __syncthreads();
-        // 3. dense part on the matrix cores (rows >= nt hold stale values and are not stored)
-        floatx16 acc;
+    } else {
+        // four chains per tile, added pairwise: shorter ones round less, and
+        // their instructions do not wait for each other
+        floatx4 part[3][2];
 #pragma unroll
-        for (int r = 0; r < 16; r++) acc[r] = 0.f;
+        for (int q = 0; q < 3; q++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(&tile[wv][c][16 * t + 8 * half]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bop[t], acc, 0, 0, 0);
+            for (int j = 0; j < 2; j++) part[q][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < 16; t++) {
+            const int k = (4 * t + lr) & (H - 1);
+            const float* W = (const float*)(t < 8 ? Sv : Nv);
+            const float a = tl[lc * PITCH + 4 * t + lr];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const float b = BACK ? W[k * H + 16 * j + lc] : W[(16 * j + lc) * H + k];
+                floatx4& to = t % 4 == 0 ? acc[j] : part[(t + 3) % 4 % 3][j];
+                to = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, to, 0, 0, 0);
+            }
         }
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int row = 8 * (r / 4) + 4 * half + (r % 4);
-            const float y = acc[r] + bias;
-            if (row < nt) hout[(tb + row) * H + c] = y > 0.f ? y : 0.f;
+        for (int j = 0; j < 2; j++) acc[j] = (acc[j] + part[0][j]) + (part[1][j] + part[2][j]);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int k = 4 * lr + v;
+        if (k >= nt) continue;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int64_t o = (i0 + k) * H + 16 * j + lc;
+            const float y = acc[j][v];
+            if constexpr (BACK) hout[o] = mask[o] > 0.f ? y : 0.f;
+            else hout[o] = y > 0.f ? y : 0.f;
         }
-        __syncthreads();
     }
 }
 
-// Output: delta_i = sigma (u_i + Wo h_i + bo), thread per unknown (nf <= kMaxNf).
-constexpr int kMaxNf = 10;
+// Output: delta_i = sigma (u_i + Wo h_i + bo), thread per unknown (nf <= kMaxNf);
+// with e1 the error left, e1 - delta, in its place.
 template <class TW>
 __global__ void k_nn_out(int n, int nf, const float* __restrict__ h, const float* __restrict__ u,
                          const TW* __restrict__ Wo, const TW* __restrict__ bo, const double* s, int slot_sigma,
-                         double* __restrict__ delta) {
+                         const double* __restrict__ e1, double* __restrict__ delta) {
     __shared__ float sWo[kMaxNf * H + kMaxNf];
     for (int e = threadIdx.x; e < nf * H; e += blockDim.x) sWo[e] = wload(Wo + e);
     if (threadIdx.x < nf) sWo[kMaxNf * H + threadIdx.x] = wload(bo + threadIdx.x);
@@ -384,104 +319,138 @@ __global__ void k_nn_out(int n, int nf, const float* __restrict__ h, const float
     float y = sWo[kMaxNf * H + a];
 #pragma unroll 8
     for (int k = 0; k < H; k++) y += sWo[a * H + k] * hi[k];
-    delta[t] = s[slot_sigma] * (double)(u[t] + y);
+    const double dl = s[slot_sigma] * (double)(u[t] + y);
+    delta[t] = e1 ? e1[t] - dl : dl;
 }
 
 // ---------------------------------------------------------------- backward
-// gy = sigma g (FP32) and dh = Wo^T gy, thread per (node, channel).
-__global__ __launch_bounds__(256) void k_nn_out_back(int n, int nf, const double* __restrict__ g,
-                                                      const double* s, int slot_sigma, const float* __restrict__ Wo,
+// g = (-2 / s[slot_e0]) Adiff, gy = sigma g (FP32), and dh = Wo^T gy where the
+// last layer's output h is positive; thread per (node, channel).
+__global__ __launch_bounds__(256) void k_nn_out_back(int n, int nf, const double* __restrict__ Adiff,
+                                                      const double* s, int slot_e0, int slot_sigma,
+                                                      const float* __restrict__ Wo, const float* __restrict__ h,
                                                       float* __restrict__ gy, float* __restrict__ dh) {
     const int c = threadIdx.x & (H - 1);
     const int64_t i = (int64_t)blockIdx.x * kNodesPerWG + (threadIdx.x >> 5);
     if (i >= n) return;
-    const double sig = s[slot_sigma];
+    const double scale = -2.0 / s[slot_e0], sig = s[slot_sigma];
     float acc = 0.f;
     for (int a = 0; a < nf; a++) {
-        const float ga = (float)(sig * g[i * nf + a]);
+        const float ga = (float)(sig * (scale * Adiff[i * nf + a]));
         if (c == 0) gy[i * nf + a] = ga;
         acc += Wo[a * H + c] * ga;
     }
-    dh[i * H + c] = acc;
+    dh[i * H + c] = h[i * H + c] > 0.f ? acc : 0.f;
 }
 
-// dpre = dh * (h > 0), in place.
-__global__ void k_nn_relu_back(int64_t count, const float* __restrict__ h, float* __restrict__ dh) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < count && !(h[t] > 0.f)) dh[t] = 0.f;
-}
+// Weight gradients of every layer: for job j (blockIdx.y) the sums over nodes
+// of A_i [B1_i B2_i]^T and of A_i, into the workgroup's share of the
+// parameters.  A has da <= 32 channels, B1 db1 <= 32, B2 none or 32.  A
+// wavefront takes 4 nodes per v_mfma_f64_16x16x4f64 step (lane l: channel
+// l % 16 of node l / 16; the products of FP32 values are exact in FP64), the
+// workgroup's wavefronts add their tiles in LDS in order.  One launch for all
+// layers: per layer and parameter matrix it was 22 us, plus 58 us for adding
+// 256 shares one after the other (11 520 nodes).
+struct NnOuterJob {
+    const float *A, *B1, *B2;
+    int da, db1;
+    int64_t o1, o2, ob;  // parameter offsets of the two matrices and the bias
+};
+constexpr int kMaxOuter = kNnMaxLayers + 2;
+struct NnOuterArgs {
+    NnOuterJob job[kMaxOuter];
+};
 
-// dprev_i = S^T dpre_i ; t_i = N^T dpre_i.
-__global__ __launch_bounds__(256) void k_nn_back_self(int n, const float* __restrict__ dpre,
-                                                       const float* __restrict__ S, const float* __restrict__ N,
-                                                       float* __restrict__ dprev, float* __restrict__ tvec) {
-    __shared__ float sS[H * H], sN[H * H];
-    __shared__ float sd[kNodesPerWG][H];
-    for (int e = threadIdx.x; e < H * H; e += blockDim.x) {
-        sS[e] = S[e];
-        sN[e] = N[e];
-    }
-    const int c = threadIdx.x & (H - 1), q = threadIdx.x >> 5;
-    const int64_t i = (int64_t)blockIdx.x * kNodesPerWG + q;
-    const bool ok = i < n;
-    sd[q][c] = ok ? dpre[i * H + c] : 0.f;
-    __syncthreads();
-    if (!ok) return;
-    float a = 0.f, b = 0.f;
-#pragma unroll 8
-    for (int k = 0; k < H; k++) {
-        a += sS[k * H + c] * sd[q][k];
-        b += sN[k * H + c] * sd[q][k];
-    }
-    dprev[i * H + c] = a;
-    tvec[i * H + c] = b;
-}
-
-// dprev_i += sum_{p in row i} wT_p t_{col(p)}  (wT_p = weight of the reverse edge).
-__global__ __launch_bounds__(256) void k_nn_back_gather(int n, const int* __restrict__ rp, const int* __restrict__ ci,
-                                                         const float* __restrict__ wT, const float* __restrict__ tvec,
-                                                         float* __restrict__ dprev) {
-    const int c = threadIdx.x & (H - 1);
-    const int64_t i = (int64_t)blockIdx.x * kNodesPerWG + (threadIdx.x >> 5);
-    if (i >= n) return;
-    float acc = 0.f;
-    for (int p = rp[i]; p < rp[i + 1]; p++) acc += wT[p] * tvec[(int64_t)ci[p] * H + c];
-    dprev[i * H + c] += acc;
-}
-
-// Partial sums over nodes of A_i B_i^T (DA x DB; B == nullptr: a column of
-// ones, i.e. the sum of A_i).  Grid of kOuterWGs workgroups, node i handled
-// by workgroup i % kOuterWGs; FP64 accumulation.
-__global__ __launch_bounds__(256) void k_nn_outer(int n, int da, int db, const float* __restrict__ Am,
-                                                   const float* __restrict__ Bm, double* __restrict__ partials) {
-    const int ne = da * db;
-    double acc[4] = {0, 0, 0, 0};
-    for (int64_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const float* a = Am + i * da;
-        const float* b = Bm ? Bm + i * db : nullptr;
+__global__ __launch_bounds__(256) void k_nn_outer(int n, int64_t np, NnOuterArgs args, double* __restrict__ partials) {
+    __shared__ double red[16 * 16];
+    const NnOuterJob J = args.job[blockIdx.y];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane >> 4, lc = lane & 15;
+    const int TB1 = (J.db1 + 15) / 16, TB2 = J.B2 ? 2 : 0, TA = (J.da + 15) / 16;
+    lane_d4 acc[2][4];
+    double sum[2] = {0.0, 0.0};
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int e = threadIdx.x + r * 256;
-            if (e < ne) {
-                const int x = e / db, y = e - x * db;
-                acc[r] += (double)a[x] * (b ? (double)b[y] : 1.0);
-            }
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) acc[a][b] = lane_d4{0.0, 0.0, 0.0, 0.0};
+    const int64_t step = (int64_t)gridDim.x * 4 * 4;
+#pragma unroll 2
+    for (int64_t i0 = ((int64_t)blockIdx.x * 4 + wave) * 4; i0 < n; i0 += step) {
+        const int64_t i = i0 + lr;
+        const bool ok = i < n;
+        double av[2], bv[4];
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            const int ch = 16 * a + lc;
+            av[a] = ok && ch < J.da ? (double)J.A[i * J.da + ch] : 0.0;
+            sum[a] += av[a];
         }
-    }
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int e = threadIdx.x + r * 256;
-        if (e < ne) partials[(int64_t)blockIdx.x * ne + e] = acc[r];
+        for (int b = 0; b < 2; b++) {
+            const int ch = 16 * b + lc;
+            bv[b] = ok && ch < J.db1 ? (double)J.B1[i * J.db1 + ch] : 0.0;
+            bv[2 + b] = ok && J.B2 ? (double)J.B2[i * H + ch] : 0.0;
+        }
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+                if (a < TA && (b < 2 ? b < TB1 : b - 2 < TB2))  // wavefront-uniform
+                    acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
     }
+    double* out = partials + (int64_t)blockIdx.x * np;
+    const int t = threadIdx.x;
+    // tile by tile: the wavefronts' sums in order
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
+            if (a >= TA || (b < 2 ? b >= TB1 : b - 2 >= TB2)) continue;  // workgroup-uniform
+            for (int w = 0; w < 4; w++) {
+                if (wave == w)
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        double* p = red + (lr + 4 * v) * 16 + lc;
+                        *p = (w > 0 ? *p : 0.0) + acc[a][b][v];
+                    }
+                __syncthreads();
+            }
+            const int x = 16 * a + t / 16, y = 16 * (b & 1) + t % 16;
+            const int db = b < 2 ? J.db1 : H;
+            if (x < J.da && y < db) out[(b < 2 ? J.o1 : J.o2) + (int64_t)x * db + y] = red[t];
+            __syncthreads();
+        }
+    // bias: nodes of the four lane rows, then the wavefronts
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        double q = sum[a];
+        q += __shfl_xor(q, 16, 64);
+        q += __shfl_xor(q, 32, 64);
+        if (lane < 16) red[wave * 32 + 16 * a + lane] = q;
+    }
+    __syncthreads();
+    if (t < J.da) out[J.ob + t] = ((red[t] + red[32 + t]) + red[64 + t]) + red[96 + t];
 }
 
-// grad[off + e] = sum over workgroups of partials (fixed order).
-__global__ void k_nn_reduce(int ne, int nwg, const double* __restrict__ partials, float* __restrict__ grad) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= ne) return;
+// grad[e] = sum over the nwg shares (fixed order): 32 parameters per
+// workgroup, 8 threads each adding every eighth share.
+__global__ __launch_bounds__(256) void k_nn_reduce(int np, int nwg, const double* __restrict__ partials,
+                                                    float* __restrict__ grad) {
+    __shared__ double sh[8][33];
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+    const int e = blockIdx.x * 32 + x;
     double s = 0;
-    for (int k = 0; k < nwg; k++) s += partials[(int64_t)k * ne + e];
-    grad[e] = (float)s;
+    if (e < np) {
+#pragma unroll 8
+        for (int k = y; k < nwg; k += 8) s += partials[(int64_t)k * np + e];
+    }
+    sh[y][x] = s;
+    __syncthreads();
+    if (y == 0 && e < np) {
+        double q = sh[0][x];
+        for (int k = 1; k < 8; k++) q += sh[k][x];
+        grad[e] = (float)q;
+    }
 }
 
 // Adam (Kingma & Ba 2015) with bias correction, and the BF16 copy of the
@@ -574,82 +543,87 @@ inline int g1(int64_t n, int bs = 256) { return (int)((n + bs - 1) / bs); }
 }  // namespace
 
 // ------------------------------------------------------------ launchers
-void nn_prep(Ctx& c, int n, int nf, const double* r1, const float* invD, float* v) {
-    hipLaunchKernelGGL(k_nn_prep, dim3(g1((int64_t)n * nf)), dim3(256), 0, c.stream, n, nf, r1, invD, v);
-    FH_HIP(hipGetLastError());
+static int prep_wgs(int n, int nf) {
+    const int R = 256 / nf;
+    return std::min((n + R - 1) / R, kPrepWGs);
 }
-void nn_input(Ctx& c, int n, int nf, const float* v, const float* feat, int slot_vv, int slot_sigma, float* u,
-              float* x0) {
-    hipLaunchKernelGGL(k_nn_input, dim3(g1((int64_t)n * (nf + 2))), dim3(256), 0, c.stream, n, nf, v, feat,
-                       c.d_scalars, slot_vv, slot_sigma, u, x0);
-    FH_HIP(hipGetLastError());
-}
-void nn_encode(Ctx& c, int n, int din, const float* x, const void* We, const void* be, bool bf16, float* h) {
-    FH_CHECK(din >= 1 && din <= kMaxDin, -3, "encoder input width out of range");
+void nn_prep(Ctx& c, int n, int nf, const double* r1, const float* invD, float* v, double* partials) {
+    FH_CHECK(nf >= 1 && nf <= kMaxNf, -3, "face block size out of range for the network");
     if (n <= 0) return;
-    const int g = (int)std::min<int64_t>(((int64_t)n + kNodesPerWG - 1) / kNodesPerWG, kEncodeMaxWGs);
-    if (bf16)
-        hipLaunchKernelGGL(k_nn_encode<bf16w>, dim3(g), dim3(256), 0, c.stream, n, din, x, (const bf16w*)We,
-                           (const bf16w*)be, h);
-    else
-        hipLaunchKernelGGL(k_nn_encode<float>, dim3(g), dim3(256), 0, c.stream, n, din, x, (const float*)We,
-                           (const float*)be, h);
+    hipLaunchKernelGGL(k_nn_prep, dim3(prep_wgs(n, nf)), dim3(256), 0, c.stream, n, nf, r1, invD, v, partials);
     FH_HIP(hipGetLastError());
 }
+void nn_encode(Ctx& c, int n, int nf, const double* partials, const float* v, const float* feat, int slot_sigma,
+               const void* We, const void* be, bool bf16, float* u, float* x0, float* h) {
+    FH_CHECK(nf >= 1 && nf <= kMaxNf, -3, "face block size out of range for the network");
+    if (n <= 0) return;
+    const int g = std::min((n + kEncodeNodes - 1) / kEncodeNodes, kEncodeMaxWGs), np = prep_wgs(n, nf);
+    if (bf16)
+        hipLaunchKernelGGL(k_nn_encode<bf16w>, dim3(g), dim3(256), 0, c.stream, n, nf, np, partials, v, feat,
+                           c.d_scalars, slot_sigma, (const bf16w*)We, (const bf16w*)be, u, x0, h);
+    else
+        hipLaunchKernelGGL(k_nn_encode<float>, dim3(g), dim3(256), 0, c.stream, n, nf, np, partials, v, feat,
+                           c.d_scalars, slot_sigma, (const float*)We, (const float*)be, u, x0, h);
+    FH_HIP(hipGetLastError());
+}
+static dim3 layer_grid(int n) { return dim3((unsigned)(((int64_t)n + kLTile * kLWaves - 1) / (kLTile * kLWaves))); }
 void nn_layer(Ctx& c, int n, const int* rp, const int* ci, const float* w, const float* hin, const void* S,
               const void* N, const void* cb, bool bf16, float* hout, float* m_out) {
-    const int g = (int)std::min<int64_t>(((int64_t)n + kLayerBatch - 1) / kLayerBatch, kLayerMaxWGs);
     if (n <= 0) return;
-    if (bf16) {
-        FH_CHECK(m_out == nullptr, -3, "the BF16 layer is inference only (no stored aggregate)");
-        int gm = (int)std::min<int64_t>(((int64_t)n + kMBatch - 1) / kMBatch, kMMaxWGs);
-        if (gm >= 64) gm -= gm % 8;  // a multiple of the XCD count selects the slab order
-        hipLaunchKernelGGL(k_nn_layer_mfma, dim3(gm), dim3(256), 0, c.stream, n, rp, ci, w, hin, (const bf16w*)S,
-                           (const bf16w*)N, (const bf16w*)cb, hout);
-    } else
-        hipLaunchKernelGGL(k_nn_layer<float>, dim3(g), dim3(256), 0, c.stream, n, rp, ci, w, hin, (const float*)S,
-                           (const float*)N, (const float*)cb, hout, m_out);
+    FH_CHECK(bf16 == (m_out == nullptr), -3, "the BF16 layer is inference only, the FP32 layer stores the aggregate");
+    if (bf16)
+        hipLaunchKernelGGL(k_nn_layer<LAYER_INFER>, layer_grid(n), dim3(kLWaves * 64), 0, c.stream, n, rp, ci, w, hin,
+                           S, N, cb, (const float*)nullptr, hout, m_out);
+    else
+        hipLaunchKernelGGL(k_nn_layer<LAYER_TRAIN>, layer_grid(n), dim3(kLWaves * 64), 0, c.stream, n, rp, ci, w, hin,
+                           S, N, cb, (const float*)nullptr, hout, m_out);
+    FH_HIP(hipGetLastError());
+}
+void nn_layer_back(Ctx& c, int n, const int* rp, const int* ci, const float* wT, const float* dpre, const float* S,
+                   const float* N, const float* h, float* dprev) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(k_nn_layer<LAYER_BACK>, layer_grid(n), dim3(kLWaves * 64), 0, c.stream, n, rp, ci, wT, dpre, S,
+                       N, (const void*)nullptr, h, dprev, (float*)nullptr);
     FH_HIP(hipGetLastError());
 }
 void nn_out(Ctx& c, int n, int nf, const float* h, const float* u, const void* Wo, const void* bo, bool bf16,
-            int slot_sigma, double* delta) {
+            int slot_sigma, const double* e1, double* delta) {
     FH_CHECK(nf >= 1 && nf <= kMaxNf, -3, "face block size out of range for the output layer");
     const int g = g1((int64_t)n * nf);
     if (bf16)
         hipLaunchKernelGGL(k_nn_out<bf16w>, dim3(g), dim3(256), 0, c.stream, n, nf, h, u, (const bf16w*)Wo,
-                           (const bf16w*)bo, c.d_scalars, slot_sigma, delta);
+                           (const bf16w*)bo, c.d_scalars, slot_sigma, e1, delta);
     else
         hipLaunchKernelGGL(k_nn_out<float>, dim3(g), dim3(256), 0, c.stream, n, nf, h, u, (const float*)Wo,
-                           (const float*)bo, c.d_scalars, slot_sigma, delta);
+                           (const float*)bo, c.d_scalars, slot_sigma, e1, delta);
     FH_HIP(hipGetLastError());
 }
-void nn_out_back(Ctx& c, int n, int nf, const double* g, int slot_sigma, const float* Wo, float* gy, float* dh) {
-    hipLaunchKernelGGL(k_nn_out_back, dim3((n + kNodesPerWG - 1) / kNodesPerWG), dim3(256), 0, c.stream, n, nf, g,
-                       c.d_scalars, slot_sigma, Wo, gy, dh);
+void nn_out_back(Ctx& c, int n, int nf, const double* Adiff, int slot_e0, int slot_sigma, const float* Wo,
+                 const float* h, float* gy, float* dh) {
+    hipLaunchKernelGGL(k_nn_out_back, dim3((n + kNodesPerWG - 1) / kNodesPerWG), dim3(256), 0, c.stream, n, nf, Adiff,
+                       c.d_scalars, slot_e0, slot_sigma, Wo, h, gy, dh);
     FH_HIP(hipGetLastError());
 }
-void nn_relu_back(Ctx& c, int64_t count, const float* h, float* dh) {
-    hipLaunchKernelGGL(k_nn_relu_back, dim3(g1(count)), dim3(256), 0, c.stream, count, h, dh);
+void nn_weight_grads(Ctx& c, int n, const NnShape& sh, const float* gy, const float* dh, const float* h,
+                     const float* m, const float* x0, double* partials, float* grad) {
+    const int64_t nH = (int64_t)n * H;
+    NnOuterArgs a{};
+    for (int l = 0; l < sh.layers; l++)
+        a.job[l] = {dh + (l + 1) * nH, h + l * nH, m + l * nH, H, H, sh.S(l), sh.N(l), sh.c(l)};
+    a.job[sh.layers] = {gy, h + sh.layers * nH, nullptr, sh.nf, H, sh.Wo(), 0, sh.bo()};
+    a.job[sh.layers + 1] = {dh, x0, nullptr, H, sh.din(), sh.We(), 0, sh.be()};
+    const int64_t np = sh.total();
+    // 4 wavefronts of 4 nodes: at least one step each, at most kOuterWGs shares
+    const int g = (int)std::min<int64_t>(std::max<int64_t>(1, ((int64_t)n + 63) / 64), kOuterWGs);
+    hipLaunchKernelGGL(k_nn_outer, dim3(g, sh.layers + 2), dim3(256), 0, c.stream, n, np, a, partials);
+    FH_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_nn_reduce, dim3((unsigned)((np + 31) / 32)), dim3(256), 0, c.stream, (int)np, g, partials,
+                       grad);
     FH_HIP(hipGetLastError());
 }
-void nn_back_self(Ctx& c, int n, const float* dpre, const float* S, const float* N, float* dprev, float* tvec) {
-    hipLaunchKernelGGL(k_nn_back_self, dim3((n + kNodesPerWG - 1) / kNodesPerWG), dim3(256), 0, c.stream, n, dpre, S,
-                       N, dprev, tvec);
-    FH_HIP(hipGetLastError());
+size_t nn_partials_bytes(const NnShape& sh) {
+    return sizeof(double) * std::max<size_t>(kPrepWGs, (size_t)kOuterWGs * sh.total());
 }
-void nn_back_gather(Ctx& c, int n, const int* rp, const int* ci, const float* wT, const float* tvec, float* dprev) {
-    hipLaunchKernelGGL(k_nn_back_gather, dim3((n + kNodesPerWG - 1) / kNodesPerWG), dim3(256), 0, c.stream, n, rp,
-                       ci, wT, tvec, dprev);
-    FH_HIP(hipGetLastError());
-}
-void nn_outer(Ctx& c, int n, int da, int db, const float* A, const float* B, double* partials, float* grad) {
-    FH_CHECK(da * db <= 1024, -3, "outer-product gradient larger than 1024 entries");
-    hipLaunchKernelGGL(k_nn_outer, dim3(kOuterWGs), dim3(256), 0, c.stream, n, da, db, A, B, partials);
-    FH_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_nn_reduce, dim3(g1(da * db)), dim3(256), 0, c.stream, da * db, kOuterWGs, partials, grad);
-    FH_HIP(hipGetLastError());
-}
-size_t nn_partials_bytes() { return sizeof(double) * kOuterWGs * 1024; }
 void nn_adam(Ctx& c, int np, float* w, const float* g, float* m1, float* m2, float lr, float b1, float b2, float eps,
              int step, void* wb) {
     const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);

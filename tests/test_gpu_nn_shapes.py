@@ -1,0 +1,47 @@
+"""Message-passing network at the edges of its tiles: fewer nodes than one
+wavefront's 16, node counts that are no multiple of 16, 64 or 128, faces with 1
+to 10 unknowns and rows of up to 11 edges (more than one batch of gathered
+neighbours).
+
+Tolerances: FP32 sums of at most 64 + 11 terms over the layers, relative to the
+largest entry: 2 * 75 * 6e-8 per layer and a condition of the output of a few
+units stay below 1e-4; the gradient passes through the layers twice."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+torch = pytest.importorskip("torch")
+F = pytest.importorskip("fhhos4_amd")
+G = F.fhgpu
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mesh,n,k,layers", [("quad", 2, 0, 1), ("quad", 2, 3, 2), ("hex", 2, 1, 2), ("hex", 2, 3, 3),
+                                             ("hex", 3, 2, 1), ("quad", 9, 1, 3), ("hex", 4, 0, 2)])
+def test_network_matches_oracle(mesh, n, k, layers):
+    print("case %s n=%d k=%d layers=%d" % (mesh, n, k, layers), flush=True)
+    ctx = G.Context(0)
+    P = G.HhoProblem(dim=3 if mesh == "hex" else 2, mesh=mesh, n=n, k=k, perturb=0.15, seed=3, kappa="lognormal",
+                     sigma=1.0)
+    A = P.matrix(ctx, keep_host=True)
+    feat = G.face_features(P)
+    g = G.NnGraph(ctx, A, feat)
+    nn = G.Mpnn(ctx, P.nf, layers=layers, seed=11)
+    rng = np.random.default_rng(6)
+    p = nn.get_params()
+    params = (p + 0.2 * rng.standard_normal(p.size)).astype(np.float32)
+    nn.set_params(params)
+    e1 = rng.standard_normal(P.n_unknowns)
+    S = P.scipy()
+    r1 = S @ e1
+    ref = O.mpnn_forward(S, P.nf, feat, params.astype(np.float64), r1, layers=layers)
+    d = torch.zeros(P.n_unknowns, dtype=torch.float64, device="cuda")
+    nn.forward(g, torch.from_numpy(r1).cuda(), d, bf16=False)
+    assert np.abs(d.cpu().numpy() - ref).max() <= 1e-4 * np.abs(ref).max()
+    nn.forward(g, torch.from_numpy(r1).cuda(), d, bf16=True)
+    assert np.linalg.norm(d.cpu().numpy() - ref) <= 3e-2 * np.linalg.norm(ref)
+    loss_ref, grad_ref = O.mpnn_loss_grad(S, P.nf, feat, params.astype(np.float64), r1, e1, layers=layers)
+    loss, grad = nn.loss_grad(g, torch.from_numpy(r1).cuda(), torch.from_numpy(e1).cuda())
+    assert abs(loss - loss_ref) <= 1e-4 * abs(loss_ref)
+    assert np.abs(grad - grad_ref).max() <= 2e-4 * np.abs(grad_ref).max()
