@@ -1,5 +1,5 @@
 // Device-side description of an HHO problem for the batched local-operator
-// and static-condensation kernel (fh_hho_kernels.hip).
+// and static-condensation kernel (fh_hho_kernels.hip, fh_hho_general.hip).
 #pragma once
 #include "fh_common.h"
 
@@ -54,8 +54,10 @@ struct HhoDev {
     const int* fexp;
 };
 
-// LDS bytes per cell (one workgroup per cell).
+// LDS bytes per affine cell (one workgroup per cell).
 size_t hho_local_lds_bytes(const HhoDev& d);
+// The general cells (kind 2) of launch_hho_local.
+void launch_hho_general(Ctx& c, const HhoDev& d);
 // Batched local operators + static condensation + scatter (vals and b must
 // be zeroed), or the post-processing mode.  Synchronises the stream.
 void launch_hho_local(Ctx& c, const HhoDev& d);
