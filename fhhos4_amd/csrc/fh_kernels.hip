@@ -751,8 +751,15 @@ __global__ void k_to_sliced(int nbr, int nslices, int W, int RW, const int* __re
 // 64 sptr[s], lane = row, so every load instruction of a wavefront reads 64
 // consecutive values and every lane has w_s independent loads to issue.
 // Padding entries hold the value 0 and the lane's own row as column.
+//
+// The coarse levels have a few wavefronts per CU, so a row's chain of
+// dependent loads (columns, then entries of x) is what the time goes to.  The
+// columns and values of the next batch are loaded before the entries of x of
+// this batch are waited for.  A Chebyshev step in FP64 takes 5.4 us on 95 232
+// rows and 4.7 us on 26 167 (7.0 us on average with batches of four loaded one
+// after the other).  The order of a row's sum is that of its slots.
 constexpr int kSellC = 64;
-constexpr int kSellUnroll = 4;
+constexpr int kSellBatch = 8;
 template <class TA, class TV, class TD, int MODE>
 __global__ __launch_bounds__(kWG) void k_sell(int nbr, int nslices, const int* __restrict__ sptr,
                                               const int* __restrict__ cols, const TA* __restrict__ sv, const TV* x,
@@ -776,27 +783,29 @@ __global__ __launch_bounds__(kWG) void k_sell(int nbr, int nslices, const int* _
         if (MODE == OP_CHEB && alpha != 0.0) dv = (AT)aux[row];
         if (MODE == OP_SPMV && beta != 0.0) yv = (AT)y[row];
     }
+    // batches of kSellBatch slots (beyond w: the last one again, not added)
     AT acc = 0;
-    int j = 0;
-    for (; j + kSellUnroll <= w; j += kSellUnroll) {
-        int c[kSellUnroll];
-        LT a[kSellUnroll];
+    int c[kSellBatch];
+    LT a[kSellBatch];
+    auto load = [&](int j) {
 #pragma unroll
-        for (int u = 0; u < kSellUnroll; u++) c[u] = cs[u * kSellC];
+        for (int u = 0; u < kSellBatch; u++) c[u] = cs[(int64_t)min(j + u, w - 1) * kSellC];
 #pragma unroll
-        for (int u = 0; u < kSellUnroll; u++) ldnt(vs + u * kSellC, a[u]);
+        for (int u = 0; u < kSellBatch; u++) ldnt(vs + (int64_t)min(j + u, w - 1) * kSellC, a[u]);
+    };
+    if (w > 0) load(0);
+    for (int j = 0; j < w; j += kSellBatch) {
+        AT xc[kSellBatch];
+        LT ac[kSellBatch];
 #pragma unroll
-        for (int u = 0; u < kSellUnroll; u++) acc += (AT)a[u] * (AT)x[c[u]];
-        cs += kSellUnroll * kSellC;
-        vs += kSellUnroll * kSellC;
-    }
-    for (; j < w; j++) {
-        LT a;
-        const int c = cs[0];
-        ldnt(vs, a);
-        acc += (AT)a * (AT)x[c];
-        cs += kSellC;
-        vs += kSellC;
+        for (int u = 0; u < kSellBatch; u++) {
+            xc[u] = (AT)x[c[u]];
+            ac[u] = a[u];
+        }
+        if (j + kSellBatch < w) load(j + kSellBatch);
+#pragma unroll
+        for (int u = 0; u < kSellBatch; u++)
+            if (j + u < w) acc += (AT)ac[u] * xc[u];
     }
     if (!out) return;
     if constexpr (MODE == OP_SPMV) {
