@@ -97,24 +97,22 @@ void launch_axpby(Ctx& c, int64_t n, Prec p, const void* x, void* y, double ha, 
 // copy when nv = 0).
 void launch_fcg_orth(Ctx& c, int64_t n, const double* z, int nv, const double* const* vs, const int* num,
                      const int* den, double* out);
-// The FP64 update fused with s[slot_rr] = <r, r> of the updated residual
-// (the value a separate launch_dots gives).
+// x += a d, r -= a q with a = s[inum] / s[iden] (CG / FCG update, FP64) and
+// s[slot_rr] = <r, r> of the updated residual
+// (the value a separate launch_dots gives).  to_host: also into c.h_scalars,
+// to be read after a synchronisation.
 void launch_cg_update_rr(Ctx& c, int64_t n, double* x, const double* d, double* r, const double* q, int inum,
-                         int iden, double sign, int slot_rr);
-// x += a d ; r -= a q with a = s[inum] / s[iden]  (CG / FCG update).
-void launch_cg_update(Ctx& c, int64_t n, Prec p, void* x, const void* d, void* r, const void* q, int inum, int iden,
-                      double sign);
+                         int iden, double sign, int slot_rr, bool to_host = false);
 // Deterministic dot products: s[slot_k] = <x_k, y_k>, k < nd (nd <= 3),
-// accumulated in FP64 with a fixed reduction tree.
-void launch_dots(Ctx& c, int64_t n, Prec p, int nd, const void* const* xs, const void* const* ys, const int* slots);
-// Device scalar arithmetic: s[dst] = op(s[a], s[b]); op 0: a/b, 1: sqrt(a),
-// 2: a*b, 3: a-b, 4: copy a.
-void launch_scalar_op(Ctx& c, int op, int dst, int a, int b);
-
-// K-cycle coefficients on the device: slots first .. first+6 hold rho1,
-// alpha1, |r|^2, |r_new|^2, gamma, beta, alpha2; ca and cb (cb = 0 when
-// |r_new| <= t |r|: the first correction alone) replace first+2, first+3.
-void launch_kcycle_coeffs(Ctx& c, int first, double t);
+// accumulated in FP64 with a fixed reduction tree; to_host as above.
+void launch_dots(Ctx& c, int64_t n, Prec p, int nd, const void* const* xs, const void* const* ys, const int* slots,
+                 bool to_host = false);
+// K-cycle: r -= (s[inum] / s[iden]) v and s[slot] = <r, r>.
+void launch_kcycle_update(Ctx& c, int64_t n, Prec p, const void* v, void* r, int inum, int iden, int slot);
+// K-cycle: slots first .. first+6 hold rho1, alpha1, |r|^2, |r_new|^2, gamma,
+// beta, alpha2; out = ca kc + cb kd (cb = 0 when |r_new| <= t |r|: the first
+// correction alone).
+void launch_kcycle_combine(Ctx& c, int64_t n, Prec p, const void* kc, const void* kd, void* out, int first, double t);
 
 // Aggregation transfers (piecewise-constant prolongation, block identity).
 // restrict: rc[I*nf+a] = sum_{k in members(I)} r[k*nf+a]

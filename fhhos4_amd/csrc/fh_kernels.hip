@@ -1022,19 +1022,6 @@ __global__ void k_fcg_orth(int64_t n, const double* z, OrthArgs p, const double*
     }
 }
 
-// Chebyshev smoothing step: d = a d + c (t - x); x = x + d, where
-// t = x + D^-1 (b - A x) was produced by the block-row kernel.
-template <class T>
-__global__ void k_cg_update(int64_t n, T* __restrict__ x, const T* __restrict__ d, T* __restrict__ r,
-                            const T* __restrict__ q, const double* s, int inum, int iden, double sign) {
-    using AT = typename Acc<T>::T;
-    const double al = sign * s[inum] / s[iden];
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
-        x[t] = (T)((AT)x[t] + (AT)al * (AT)d[t]);
-        r[t] = (T)((AT)r[t] - (AT)al * (AT)q[t]);
-    }
-}
-
 template <int ND>
 __device__ __forceinline__ void block_reduce(double (&v)[3], double* sh) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -1056,6 +1043,14 @@ __device__ __forceinline__ void block_reduce(double (&v)[3], double* sh) {
         }
     }
 }
+
+// Where a reduction's results go: slots of s and, with host (pinned), a copy
+// that the program reads after a synchronisation without a copy of its own.
+struct DotOut {
+    double* s;
+    double* host;
+    int slot[3];
+};
 
 // SX: every product has the same x (read once; the products and sums are
 // those of separate x reads)
@@ -1095,39 +1090,58 @@ __global__ __launch_bounds__(kWG) void k_cg_update_rr(int64_t n, double* __restr
     if (threadIdx.x == 0) partials[blockIdx.x] = v[0];
 }
 
+// K-cycle: r <- r - (s[inum] / s[iden]) v and |r|^2 of the stored result, the
+// arithmetic of k_axpby, then of k_dots on the same grid, in one pass.
+template <class T>
+__global__ __launch_bounds__(kWG) void k_kcycle_update(int64_t n, const T* __restrict__ v, T* __restrict__ r,
+                                                       const double* s, int inum, int iden, double* partials) {
+#pragma clang fp contract(off)
+    using AT = typename Acc<T>::T;
+    __shared__ double sh[3 * 16];
+    const AT a = (AT)scal(s, -1.0, inum, iden);
+    double p[3] = {0, 0, 0};
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
+        const AT av = a * (AT)v[t];
+        const T rn = (T)(av + (AT)r[t]);
+        r[t] = rn;
+        p[0] = fma((double)rn, (double)rn, p[0]);
+    }
+    block_reduce<1>(p, sh);
+    if (threadIdx.x == 0) partials[blockIdx.x] = p[0];
+}
+
+// Sums of nb workgroups' partials (a reduction that the last workgroup to
+// arrive finishes in the same launch was slower: 9.6 us for 103 workgroups
+// and 20.6 us for 1024, where the two launches take 8.4 us and 9.3 us; the
+// arrivals are serial accesses across the XCDs).
 template <int ND>
-__global__ __launch_bounds__(1024) void k_dots_final(const double* partials, double* s, int s0, int s1, int s2) {
+__global__ __launch_bounds__(1024) void k_dots_final(const double* partials, int nb, DotOut o) {
     __shared__ double sh[3 * 16];
     double v[3] = {0, 0, 0};
     const int t = threadIdx.x;
-    for (int k = 0; k < ND; k++) v[k] = partials[k * kDotBlocks + t];
+    if (t < nb)
+        for (int k = 0; k < ND; k++) v[k] = partials[k * kDotBlocks + t];
     block_reduce<ND>(v, sh);
-    if (t == 0) {
-        s[s0] = v[0];
-        if (ND > 1) s[s1] = v[1];
-        if (ND > 2) s[s2] = v[2];
-    }
+    if (t == 0)
+        for (int k = 0; k < ND; k++) {
+            o.s[o.slot[k]] = v[k];
+            if (o.host) o.host[o.slot[k]] = v[k];
+        }
 }
 
-__global__ void k_scalar_op(double* s, int op, int dst, int a, int b) {
-    double r = 0;
-    switch (op) {
-        case 0: r = s[a] / s[b]; break;
-        case 1: r = sqrt(s[a]); break;
-        case 2: r = s[a] * s[b]; break;
-        case 3: r = s[a] - s[b]; break;
-        default: r = s[a]; break;
-    }
-    s[dst] = r;
-}
-
-// Coefficients of the K-cycle's FCG step (Multigrid::FCGForKCycle,
-// Multigrid.h:611-656) from the device slots s[k .. k+6] = rho1, alpha1,
-// |r|^2, |r_new|^2, gamma, beta, alpha2: when |r_new| <= t |r| the first
-// correction alone is kept (ca = alpha1 / rho1, cb = 0), else
-// rho2 = beta - gamma^2 / rho1, ca = alpha1 / rho1 - gamma alpha2 / (rho1 rho2),
-// cb = alpha2 / rho2.  ca and cb replace s[k+2] and s[k+3].
-__global__ void k_kcycle_coeffs(double* s, int k, double t) {
+// The result out = ca c + cb d of the K-cycle's FCG step
+// (Multigrid::FCGForKCycle, Multigrid.h:611-656) from the device slots
+// s[k .. k+6] = rho1, alpha1, |r|^2, |r_new|^2, gamma, beta, alpha2: when
+// |r_new| <= t |r| the first correction alone is kept (ca = alpha1 / rho1,
+// cb = 0), else rho2 = beta - gamma^2 / rho1,
+// ca = alpha1 / rho1 - gamma alpha2 / (rho1 rho2), cb = alpha2 / rho2.
+// Every thread forms the two coefficients; products and sums are rounded one
+// by one.  (A launch for the coefficients and one for each product before.)
+template <class T>
+__global__ void k_kcycle_combine(int64_t n, const T* __restrict__ c, const T* __restrict__ d, T* __restrict__ out,
+                                 const double* s, int k, double t) {
+#pragma clang fp contract(off)
+    using AT = typename Acc<T>::T;
     const double rho1 = s[k], alpha1 = s[k + 1], rold = sqrt(s[k + 2]), rnew = sqrt(s[k + 3]);
     double ca, cb;
     if (rnew <= t * rold) {
@@ -1135,12 +1149,15 @@ __global__ void k_kcycle_coeffs(double* s, int k, double t) {
         cb = 0.0;
     } else {
         const double gamma = s[k + 4], beta = s[k + 5], alpha2 = s[k + 6];
-        const double rho2 = __dsub_rn(beta, __ddiv_rn(__dmul_rn(gamma, gamma), rho1));
-        ca = __dsub_rn(__ddiv_rn(alpha1, rho1), __ddiv_rn(__dmul_rn(gamma, alpha2), __dmul_rn(rho1, rho2)));
+        const double rho2 = beta - gamma * gamma / rho1;
+        ca = alpha1 / rho1 - gamma * alpha2 / (rho1 * rho2);
         cb = alpha2 / rho2;
     }
-    s[k + 2] = ca;
-    s[k + 3] = cb;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const T oc = (T)((AT)ca * (AT)c[i]);
+    const AT od = (AT)cb * (AT)d[i];
+    out[i] = (T)(od + (AT)oc);
 }
 
 template <class T>
@@ -2102,42 +2119,41 @@ void launch_fcg_orth(Ctx& c, int64_t n, const double* z, int nv, const double* c
     }
 }
 
+template <int ND>
+static void dots_final(Ctx& c, int nb, const int* slots, bool to_host) {
+    DotOut o{c.d_scalars, to_host ? c.h_scalars : nullptr, {0, 0, 0}};
+    for (int k = 0; k < ND; k++) o.slot[k] = slots[k];
+    hipLaunchKernelGGL((k_dots_final<ND>), dim3(1), dim3(kDotBlocks), 0, c.stream, c.d_partials, nb, o);
+    FH_HIP(hipGetLastError());
+}
+// one entry per thread up to kDotBlocks workgroups (empty ones add nothing)
+static int dot_grid(int64_t n) { return (int)std::min<int64_t>(kDotBlocks, std::max<int64_t>(1, (n + kWG - 1) / kWG)); }
+
 void launch_cg_update_rr(Ctx& c, int64_t n, double* x, const double* d, double* r, const double* q, int inum,
-                         int iden, double sign, int slot_rr) {
+                         int iden, double sign, int slot_rr, bool to_host) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_cg_update_rr, dim3(kDotBlocks), dim3(kWG), 0, c.stream, n, x, d, r, q, c.d_scalars, inum, iden,
-                       sign, c.d_partials);
-    hipLaunchKernelGGL((k_dots_final<1>), dim3(1), dim3(kDotBlocks), 0, c.stream, c.d_partials, c.d_scalars, slot_rr, 0,
-                       0);
+    const int g = dot_grid(n);
+    hipLaunchKernelGGL(k_cg_update_rr, dim3(g), dim3(kWG), 0, c.stream, n, x, d, r, q, c.d_scalars, inum, iden, sign,
+                       c.d_partials);
     FH_HIP(hipGetLastError());
+    dots_final<1>(c, g, &slot_rr, to_host);
 }
 
-void launch_cg_update(Ctx& c, int64_t n, Prec p, void* x, const void* d, void* r, const void* q, int inum, int iden,
-                      double sign) {
-    if (n <= 0) return;
-    int g = grid_for(n);
-    if (p == Prec::F64)
-        hipLaunchKernelGGL((k_cg_update<double>), dim3(g), dim3(256), 0, c.stream, n, (double*)x, (const double*)d,
-                           (double*)r, (const double*)q, c.d_scalars, inum, iden, sign);
-    else
-        hipLaunchKernelGGL((k_cg_update<float>), dim3(g), dim3(256), 0, c.stream, n, (float*)x, (const float*)d,
-                           (float*)r, (const float*)q, c.d_scalars, inum, iden, sign);
-    FH_HIP(hipGetLastError());
-}
-
-void launch_dots(Ctx& c, int64_t n, Prec p, int nd, const void* const* xs, const void* const* ys, const int* slots) {
+void launch_dots(Ctx& c, int64_t n, Prec p, int nd, const void* const* xs, const void* const* ys, const int* slots,
+                 bool to_host) {
     FH_CHECK(nd >= 1 && nd <= 3, -3, "1 to 3 dot products per launch");
     const void* X[3] = {xs[0], nd > 1 ? xs[1] : xs[0], nd > 2 ? xs[2] : xs[0]};
     const void* Y[3] = {ys[0], nd > 1 ? ys[1] : ys[0], nd > 2 ? ys[2] : ys[0]};
     const bool sx = X[1] == X[0] && X[2] == X[0];
+    const int g = dot_grid(n);
 #define FH_DOTS(T, ND)                                                                                              \
     do {                                                                                                            \
         if (sx)                                                                                                     \
-            hipLaunchKernelGGL((k_dots<T, ND, true>), dim3(kDotBlocks), dim3(kWG), 0, c.stream, n, (const T*)X[0],   \
+            hipLaunchKernelGGL((k_dots<T, ND, true>), dim3(g), dim3(kWG), 0, c.stream, n, (const T*)X[0],            \
                                (const T*)Y[0], (const T*)X[1], (const T*)Y[1], (const T*)X[2], (const T*)Y[2],       \
                                c.d_partials);                                                                       \
         else                                                                                                        \
-            hipLaunchKernelGGL((k_dots<T, ND, false>), dim3(kDotBlocks), dim3(kWG), 0, c.stream, n, (const T*)X[0],  \
+            hipLaunchKernelGGL((k_dots<T, ND, false>), dim3(g), dim3(kWG), 0, c.stream, n, (const T*)X[0],           \
                                (const T*)Y[0], (const T*)X[1], (const T*)Y[1], (const T*)X[2], (const T*)Y[2],       \
                                c.d_partials);                                                                       \
     } while (0)
@@ -2147,20 +2163,34 @@ void launch_dots(Ctx& c, int64_t n, Prec p, int nd, const void* const* xs, const
         if (nd == 1) FH_DOTS(float, 1); else if (nd == 2) FH_DOTS(float, 2); else FH_DOTS(float, 3);
     }
 #undef FH_DOTS
-    int s0 = slots[0], s1 = nd > 1 ? slots[1] : 0, s2 = nd > 2 ? slots[2] : 0;
-    if (nd == 1) hipLaunchKernelGGL((k_dots_final<1>), dim3(1), dim3(kDotBlocks), 0, c.stream, c.d_partials, c.d_scalars, s0, s1, s2);
-    else if (nd == 2) hipLaunchKernelGGL((k_dots_final<2>), dim3(1), dim3(kDotBlocks), 0, c.stream, c.d_partials, c.d_scalars, s0, s1, s2);
-    else hipLaunchKernelGGL((k_dots_final<3>), dim3(1), dim3(kDotBlocks), 0, c.stream, c.d_partials, c.d_scalars, s0, s1, s2);
     FH_HIP(hipGetLastError());
+    if (nd == 1) dots_final<1>(c, g, slots, to_host);
+    else if (nd == 2) dots_final<2>(c, g, slots, to_host);
+    else dots_final<3>(c, g, slots, to_host);
 }
 
-void launch_scalar_op(Ctx& c, int op, int dst, int a, int b) {
-    hipLaunchKernelGGL(k_scalar_op, dim3(1), dim3(1), 0, c.stream, c.d_scalars, op, dst, a, b);
+void launch_kcycle_update(Ctx& c, int64_t n, Prec p, const void* v, void* r, int inum, int iden, int slot) {
+    if (n <= 0) return;
+    const int g = dot_grid(n);
+    if (p == Prec::F64)
+        hipLaunchKernelGGL((k_kcycle_update<double>), dim3(g), dim3(kWG), 0, c.stream, n, (const double*)v, (double*)r,
+                           c.d_scalars, inum, iden, c.d_partials);
+    else
+        hipLaunchKernelGGL((k_kcycle_update<float>), dim3(g), dim3(kWG), 0, c.stream, n, (const float*)v, (float*)r,
+                           c.d_scalars, inum, iden, c.d_partials);
     FH_HIP(hipGetLastError());
+    dots_final<1>(c, g, &slot, false);
 }
 
-void launch_kcycle_coeffs(Ctx& c, int first, double t) {
-    hipLaunchKernelGGL(k_kcycle_coeffs, dim3(1), dim3(1), 0, c.stream, c.d_scalars, first, t);
+void launch_kcycle_combine(Ctx& c, int64_t n, Prec p, const void* kc, const void* kd, void* out, int first, double t) {
+    if (n <= 0) return;
+    const dim3 g((unsigned)((n + 255) / 256));
+    if (p == Prec::F64)
+        hipLaunchKernelGGL((k_kcycle_combine<double>), g, dim3(256), 0, c.stream, n, (const double*)kc,
+                           (const double*)kd, (double*)out, c.d_scalars, first, t);
+    else
+        hipLaunchKernelGGL((k_kcycle_combine<float>), g, dim3(256), 0, c.stream, n, (const float*)kc, (const float*)kd,
+                           (float*)out, c.d_scalars, first, t);
     FH_HIP(hipGetLastError());
 }
 

@@ -134,24 +134,18 @@ Ctx::~Ctx() {
     count_context(-1);
 }
 
-static void read_scalars(Ctx& c, int first, int count) {
-    FH_HIP(hipMemcpyAsync(c.h_scalars + first, c.d_scalars + first, sizeof(double) * count, hipMemcpyDeviceToHost,
-                          c.stream));
-    FH_HIP(hipStreamSynchronize(c.stream));
-}
-
-static void dot1(Ctx& c, int64_t n, Prec p, const void* x, const void* y, int slot) {
+static void dot1(Ctx& c, int64_t n, Prec p, const void* x, const void* y, int slot, bool to_host = false) {
     const void* xs[1] = {x};
     const void* ys[1] = {y};
     int sl[1] = {slot};
-    launch_dots(c, n, p, 1, xs, ys, sl);
+    launch_dots(c, n, p, 1, xs, ys, sl, to_host);
 }
 static void dot2(Ctx& c, int64_t n, Prec p, const void* x0, const void* y0, int s0, const void* x1, const void* y1,
-                 int s1) {
+                 int s1, bool to_host = false) {
     const void* xs[2] = {x0, x1};
     const void* ys[2] = {y0, y1};
     int sl[2] = {s0, s1};
-    launch_dots(c, n, p, 2, xs, ys, sl);
+    launch_dots(c, n, p, 2, xs, ys, sl, to_host);
 }
 static void dot3(Ctx& c, int64_t n, Prec p, const void* x0, const void* y0, int s0, const void* x1, const void* y1,
                  int s1, const void* x2, const void* y2, int s2) {
@@ -211,8 +205,8 @@ double estimate_lmax(Ctx& c, const Bcsr& A64, const void* invD64) {
                     nullptr, 0);
         FH_HIP(hipMemcpyAsync(w.data(), v.data(), sizeof(double) * n, hipMemcpyDeviceToDevice, c.stream));
         launch_axpby(c, n, Prec::F64, t.data(), w.data(), -1.0, -1, -1, 1.0, -1, -1);
-        dot2(c, n, Prec::F64, w.data(), w.data(), slot, v.data(), v.data(), slot + 1);
-        read_scalars(c, slot, 2);
+        dot2(c, n, Prec::F64, w.data(), w.data(), slot, v.data(), v.data(), slot + 1, true);
+        c.sync();
         const double nw = std::sqrt(c.h_scalars[slot]), nv = std::sqrt(c.h_scalars[slot + 1]);
         FH_CHECK(nw > 0 && nv > 0, -6, "power iteration met a zero vector");
         lam = nw / nv;
@@ -697,15 +691,12 @@ public:
         cycle(l, r.data(), V.kc, true, &V.kv);
         // rho1 = c.v, alpha1 = c.r, |r|^2
         dot3(c_, V.n, vp_, V.kc.data(), V.kv.data(), s + 0, V.kc.data(), r.data(), s + 1, r.data(), r.data(), s + 2);
-        // r <- r - (alpha1 / rho1) v, then |r_new|^2
-        launch_axpby(c_, V.n, vp_, V.kv.data(), r.data(), -1.0, s + 1, s + 0, 1.0, -1, -1);
-        dot1(c_, V.n, vp_, r.data(), r.data(), s + 3);
+        // r <- r - (alpha1 / rho1) v and |r_new|^2
+        launch_kcycle_update(c_, V.n, vp_, V.kv.data(), r.data(), s + 1, s + 0, s + 3);
         cycle(l, r.data(), V.kd, true, &V.kw);
         // gamma = d.v, beta = d.w, alpha2 = d.r
         dot3(c_, V.n, vp_, V.kd.data(), V.kv.data(), s + 4, V.kd.data(), V.kw.data(), s + 5, V.kd.data(), r.data(), s + 6);
-        launch_kcycle_coeffs(c_, s, t);
-        launch_axpby(c_, V.n, vp_, V.kc.data(), out.data(), 1.0, s + 2, -1, 0.0, -1, -1);
-        launch_axpby(c_, V.n, vp_, V.kd.data(), out.data(), 1.0, s + 3, -1, 1.0, -1, -1);
+        launch_kcycle_combine(c_, V.n, vp_, V.kc.data(), V.kd.data(), out.data(), s, t);
     }
 };
 
@@ -916,8 +907,9 @@ void Solver::ApplyPreconditioner(const double* r, double* z) {
     c_.sync();
 }
 
+// The scalar that a reduction launched with to_host left.
 double Solver::read_scalar(int slot) {
-    read_scalars(c_, slot, 1);
+    c_.sync();
     return c_.h_scalars[slot];
 }
 
@@ -1021,7 +1013,7 @@ double Solver::initial_residual(const double* b, double* x, bool xz, double& res
     } else {
         launch_bcsr(c_, *A_, OP_RESID, P, x, b, r_.data(), 1.0, 0.0, 0.0, nullptr, P, nullptr, 0);
     }
-    dot2(c_, n, P, b, b, S_BB, r_.data(), r_.data(), S_RR);
+    dot2(c_, n, P, b, b, S_BB, r_.data(), r_.data(), S_RR, true);
     const double bn = std::sqrt(read_scalar(S_BB));
     const double rn = std::sqrt(read_scalar(S_RR));
     res = xz ? 1.0 : (bn > 0 ? rn / bn : rn);
@@ -1036,20 +1028,30 @@ void Solver::solve_cg(const double* b, double* x, bool xz) {
     const double bn = initial_residual(b, x, xz, res);
     apply_prec(r_, z_, nullptr);
     copy(c_, n, P, z_.data(), d_.data());
-    dot1(c_, n, P, r_.data(), z_.data(), S_RZ);
+    // r . z of this iteration and of the one before take turns in two slots
+    const int rz[2] = {S_RZ, S_RZOLD};
+    dot1(c_, n, P, r_.data(), z_.data(), rz[0]);
     int it = 0;
     hist_.push_back(res);
     stats_.converged = 0;
     auto stop = FH_STOP_TEST();
+    auto precondition = [&] {
+        apply_prec(r_, z_, nullptr);
+        dot1(c_, n, P, r_.data(), z_.data(), rz[it % 2]);
+    };
     while (!stop()) {
-        if (it > 0) launch_axpby(c_, n, P, z_.data(), d_.data(), 1.0, -1, -1, 1.0, S_RZ, S_RZOLD);  // d = z + beta d
+        if (it > 0) {
+            if (!nn_) precondition();
+            launch_axpby(c_, n, P, z_.data(), d_.data(), 1.0, -1, -1, 1.0, rz[it % 2], rz[(it + 1) % 2]);  // d = z + beta d
+        }
         launch_bcsr(c_, *A_, OP_SPMV, P, d_.data(), nullptr, Ad_.data(), 1.0, 0.0, 0.0, nullptr, P, nullptr, 0);
         dot1(c_, n, P, d_.data(), Ad_.data(), S_DAD);
-        launch_cg_update(c_, n, P, x, d_.data(), r_.data(), Ad_.data(), S_RZ, S_DAD, 1.0);
-        launch_scalar_op(c_, 4, S_RZOLD, S_RZ, 0);
-        apply_prec(r_, z_, nullptr);
-        dot2(c_, n, P, r_.data(), z_.data(), S_RZ, r_.data(), r_.data(), S_RR);
+        launch_cg_update_rr(c_, n, (double*)x, (const double*)d_.data(), (double*)r_.data(), (const double*)Ad_.data(),
+                            rz[it % 2], S_DAD, 1.0, S_RR, true);
         it++;
+        // |r| decides before the next preconditioner application, except that
+        // the learned post-smoother counts one after the last iteration too
+        if (nn_) precondition();
         double rr = read_scalar(S_RR);
         res = bn > 0 ? std::sqrt(rr) / bn : std::sqrt(rr);
         hist_.push_back(res);
@@ -1137,15 +1139,14 @@ void Solver::solve_fcg(const double* b, double* x, bool xz) {
         }
         since_replace = approx ? since_replace + 1 : since_replace;
         // d.Ad and d.r (= r.d) in one pass over d
-        dot2(c_, n, P, d.data(), Ad.data(), S_DAD, d.data(), r_.data(), S_RD);
+        dot2(c_, n, P, d.data(), Ad.data(), slot_dad(cur), d.data(), r_.data(), S_RD);
         // x += a d, r -= a Ad and |r|^2 in one pass
         launch_cg_update_rr(c_, n, x, (const double*)d.data(), (double*)r_.data(), (const double*)Ad.data(), S_RD,
-                            S_DAD, 1.0, S_RR);
+                            slot_dad(cur), 1.0, S_RR, true);
         if ((int)kept.size() == m) {
             if (args_.fcg_restart) kept.clear();
             else kept.erase(kept.begin());
         }
-        launch_scalar_op(c_, 4, slot_dad(cur), S_DAD, 0);
         kept.push_back(cur);
         it++;
         double rr = read_scalar(S_RR);
@@ -1155,7 +1156,7 @@ void Solver::solve_fcg(const double* b, double* x, bool xz) {
             // rounding of the FP32-stored products; the stopping test and the
             // next directions use the FP64 b - A x
             launch_bcsr(c_, *A_, OP_RESID, P, x, b, r_.data(), 1.0, 0.0, 0.0, nullptr, P, nullptr, 0);
-            dot1(c_, n, P, r_.data(), r_.data(), S_RR);
+            dot1(c_, n, P, r_.data(), r_.data(), S_RR, true);
             rr = read_scalar(S_RR);
             res = bn > 0 ? std::sqrt(rr) / bn : std::sqrt(rr);
             since_replace = 0;
@@ -1185,7 +1186,7 @@ void Solver::solve_stationary(const double* b, double* x, bool xz) {
             copy(c_, n, P, z_.data(), x);
         }
         launch_bcsr(c_, *A_, OP_RESID, P, x, b, r_.data(), 1.0, 0.0, 0.0, nullptr, P, nullptr, 0);
-        dot1(c_, n, P, r_.data(), r_.data(), S_RR);
+        dot1(c_, n, P, r_.data(), r_.data(), S_RR, true);
         it++;
         double rr = read_scalar(S_RR);
         res = bn > 0 ? std::sqrt(rr) / bn : std::sqrt(rr);
