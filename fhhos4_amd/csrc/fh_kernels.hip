@@ -309,7 +309,6 @@ template <class T> __device__ __forceinline__ void ldnt4(const T*, float&, float
 // buffer resource: 32-bit data format, no swizzle.
 constexpr int kBufferWord3 = 0x00020000;
 constexpr int kBufferNt = 2;  // cache policy bits of the load: non-temporal
-template <class T> constexpr bool kRawSliceLoads = std::is_same<T, double>::value || std::is_same<T, float>::value;
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void ldbuf2(__amdgpu_buffer_rsrc_t r, int voff, int soff, double& a, double& b) {
@@ -329,8 +328,27 @@ __device__ __forceinline__ void ldbuf1(__amdgpu_buffer_rsrc_t r, int voff, int s
 __device__ __forceinline__ void ldbuf1(__amdgpu_buffer_rsrc_t r, int voff, int soff, float& a) {
     a = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, kBufferNt));
 }
-template <class T> __device__ __forceinline__ void ldbuf2(__amdgpu_buffer_rsrc_t, int, int, float&, float&) {}
-template <class T> __device__ __forceinline__ void ldbuf1(__amdgpu_buffer_rsrc_t, int, int, float&) {}
+// Values of a slice as they are loaded (CW per lane), widened at their use:
+// a BF16 pair stays one word until then, so that no conversion waits for the
+// loads before the ones behind them are issued.
+template <class TA, int CW> struct SliceValue {
+    TA v[CW];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int lane, int off) {
+        if constexpr (CW == 2) ldbuf2(r, lane * 2 * (int)sizeof(TA), off * 2 * (int)sizeof(TA), v[0], v[1]);
+        else ldbuf1(r, lane * (int)sizeof(TA), off * (int)sizeof(TA), v[0]);
+    }
+    __device__ __forceinline__ TA get(int j) const { return v[j]; }
+};
+template <int CW> struct SliceValue<bf16_t, CW> {
+    uint32_t u;
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int lane, int off) {
+        if constexpr (CW == 2) u = __builtin_amdgcn_raw_buffer_load_b32(r, lane * 4, off * 4, kBufferNt);
+        else u = (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, lane * 2, off * 2, kBufferNt);
+    }
+    __device__ __forceinline__ float get(int j) const {
+        return __uint_as_float(j == 0 ? u << 16 : u & 0xffff0000u);
+    }
+};
 
 constexpr int kSlicedWaves = kWG / 64;  // slices per workgroup
 
@@ -343,7 +361,15 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Block-row operation on the sliced layout (all rows), one slice per
+// n / d for n < 64, d <= 64 by rcp = small_rcp(d)
+constexpr unsigned small_rcp(int d) { return (65536u + d - 1) / d; }
+__device__ __forceinline__ unsigned small_div(unsigned n, unsigned rcp) { return __umul24(n, rcp) >> 16; }
+
+// partial sums of a wavefront in LDS: row pitch, and how many are loaded
+// before the first is added (reads may run that far past a row)
+constexpr int kRedPitch = 65, kRedBatch = 8;
+
+// Block-row operation on the sliced layout (all rows), NS slices per
 // wavefront.  Lane (r, b, jp) multiplies column group jp of block slot b of
 // row r by its x entries, for the NF rows i of the block; the NF partial
 // sums per lane go to LDS and 64 / (RW * NF) lanes per (r, i) add the
@@ -356,10 +382,17 @@ __device__ __forceinline__ void wave_lds_sync() {
 // block r) when RW * NF * JP <= 64, and D^-1 times the residual is then
 // summed with shuffles.  MAP: the rows of this part are rowmap[0 .. nbr)
 // (else 0 .. nbr).
-template <int NF, class TA, class TV, class TD, int MODE, bool MAP>
-__global__ __launch_bounds__(kWG) void k_sliced(int nbr, int nslices, int W, int RW, const int* __restrict__ cols,
-                                                const TA* __restrict__ sv, const TV* x, const TV* b, TV* y,
-                                                double alpha, double beta, double omega,
+//
+// A slice of 64 lanes holds 1 to 3 KB of values, so the instructions around
+// the loads count as much as the bytes: lane indexes come from multiplications
+// by reciprocals, entries are addressed from the slice's first one, and the
+// partial sums are read from LDS several at a time.  The residual of 142 876
+// block rows of n_f = 6 in BF16 (76 MB) takes 16.8 us, 24.6 us with runtime
+// divisions, one slice per wavefront and sums read one by one.
+template <int NF, class TA, class TV, class TD, int MODE, bool MAP, int NS>
+__global__ __launch_bounds__(kWG) void k_sliced(int nbr, int nslices, int W, int RW, int rcp, int lognp,
+                                                const int* __restrict__ cols, const TA* __restrict__ sv, const TV* x,
+                                                const TV* b, TV* y, double alpha, double beta, double omega,
                                                 const TD* __restrict__ invD, TV* __restrict__ aux,
                                                 const int* __restrict__ rowmap) {
     using AT = typename Acc<TV>::T;
@@ -367,148 +400,169 @@ __global__ __launch_bounds__(kWG) void k_sliced(int nbr, int nslices, int W, int
     constexpr int JP = NF / CW;
     constexpr bool SMOOTHING = MODE == OP_CHEB || MODE == OP_SMOOTH;
     const int LPR = W * JP, ACT = RW * LPR;
-    __shared__ AT red[kSlicedWaves][NF][64];
+    __shared__ AT red[kSlicedWaves][NF * kRedPitch + kRedBatch + 32];  // reads run at most 36 past the rows
     // the wavefront index as a uniform value: slice offsets stay scalar
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int s = xcd_remap(blockIdx.x, gridDim.x) * kSlicedWaves + wave;
-    if (s >= nslices) return;  // wavefront-uniform; no workgroup barrier follows
+    const unsigned lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int s0 = (xcd_remap(blockIdx.x, gridDim.x) * kSlicedWaves + wave) * NS;
+    if (s0 >= nslices) return;  // wavefront-uniform; no workgroup barrier follows
 
     // product lane (rv, bs, jp)
-    const int rv = lane / LPR, rl = lane - rv * LPR, bs = rl / JP, jp = rl - bs * JP;
-    const bool act = lane < ACT;
-    const int c = act ? cols[(int64_t)s * RW * W + rv * W + bs] : -1;
-    // loaded value type: FP64 values load as doubles, FP32 and BF16 ones as
-    // floats (widened to the accumulation type at use)
-    using LT = std::conditional_t<std::is_same<TA, double>::value, double, float>;
-    LT a[NF][CW];
-    if (act) {
+    const unsigned rv = small_div(lane, (unsigned)rcp), rl = lane - __umul24(rv, LPR),
+                   bs = small_div(rl, small_rcp(JP)), jp = rl - __umul24(bs, JP);
+    const bool act = lane < (unsigned)ACT;
+    const unsigned co = __umul24(rv, W) + bs;
+    int c[NS];
+#pragma unroll
+    for (int u = 0; u < NS; u++)
+        c[u] = act && s0 + u < nslices ? (cols + (int64_t)(s0 + u) * RW * W)[co] : -1;
+    SliceValue<TA, CW> a[NS][NF];
+#pragma unroll
+    for (int u = 0; u < NS; u++) {
+        const int s = s0 + u;
+        if (!act || s >= nslices) continue;
         // The slice's value loads: its base in a buffer resource (scalar
         // registers), the row offset scalar, the lane offset one VGPR.
         // Padding slots hold zero values.
         const TA* sbase = sv + (int64_t)s * NF * ACT * CW;
-        if constexpr (kRawSliceLoads<TA>) {
-            const auto rs =
-                __builtin_amdgcn_make_buffer_rsrc((void*)sbase, 0, (int)(NF * ACT * CW * sizeof(TA)), kBufferWord3);
+        const auto rs =
+            __builtin_amdgcn_make_buffer_rsrc((void*)sbase, 0, (int)(NF * ACT * CW * sizeof(TA)), kBufferWord3);
 #pragma unroll
-            for (int k = 0; k < NF; k++) {
-                if constexpr (CW == 2)
-                    ldbuf2(rs, lane * CW * (int)sizeof(TA), k * ACT * CW * (int)sizeof(TA), a[k][0], a[k][1]);
-                else
-                    ldbuf1(rs, lane * (int)sizeof(TA), k * ACT * (int)sizeof(TA), a[k][0]);
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < NF; k++) {
-                if constexpr (CW == 2)
-                    ldnt2(sbase + (int64_t)k * ACT * 2 + lane * 2, a[k][0], a[k][1]);
-                else
-                    ldnt(sbase + (int64_t)k * ACT + lane, a[k][0]);
-            }
-        }
+        for (int k = 0; k < NF; k++) a[u][k].load(rs, (int)lane, k * ACT);
     }
 
     // output lane (r, i, part 0) of row r, entry i; parts 1 .. NP - 1 (NP a
     // power of two) help to sum
-    const int NP = 1 << (31 - __clz(64 / (RW * NF)));
-    const int r = lane / (NF * NP), rem = lane - r * (NF * NP), i = rem % NF, part = rem / NF;
-    const int row = s * RW + r;
-    const bool out = r < RW && part == 0 && row < nbr;  // nbr: rows of this part
-    const int64_t e = (int64_t)(MAP && out ? rowmap[row] : row) * NF + i;
-    AT bv = 0, xv = 0, dv = 0, yv = 0;
-    if (out) {
-        if (MODE != OP_SPMV) bv = (AT)b[e];
-        if (SMOOTHING) xv = (AT)x[e];
-        if (MODE == OP_CHEB && alpha != 0.0) dv = (AT)aux[e];
-        if (MODE == OP_SPMV && beta != 0.0) yv = (AT)y[e];
-    }
+    const unsigned t = small_div(lane, small_rcp(NF)), r = t >> lognp, part = t & ((1u << lognp) - 1), i = lane - __umul24(t, NF);
     // inverse-block lane (dr, di, dm)
     const bool dist = SMOOTHING && RW * NF * JP <= 64;
-    const bool dlane = dist && lane < RW * NF * JP;
-    const int dr = dlane ? lane / (NF * JP) : 0;
-    const int di = dlane ? (lane - dr * (NF * JP)) / JP : 0;
-    const int dm = dlane ? lane - dr * (NF * JP) - di * JP : 0;
-    AT d0 = 0, d1 = 0;
-    const int drow = s * RW + dr;
-    if (dlane && drow < nbr) {
-        const TD* D = invD + ((int64_t)(MAP ? rowmap[drow] : drow) * NF + di) * NF + CW * dm;
-        d0 = (AT)ldv(D);
-        if constexpr (CW == 2) d1 = (AT)ldv(D + 1);
+    const bool dlane = dist && lane < (unsigned)(RW * NF * JP);
+    const unsigned dt = small_div(lane, small_rcp(JP)), dm = lane - __umul24(dt, JP),
+                   dr = small_div(dt, small_rcp(NF)), di = dt - __umul24(dr, NF);
+    // offsets of the lane's output entry and inverse-block entries from those
+    // of the slice (MAP: of the row)
+    const unsigned eo = MAP ? i : __umul24(r, NF) + i, doff = __umul24(MAP ? di : dt, NF) + CW * dm;
+    const bool orow = r < (unsigned)RW && part == 0;
+    AT bv[NS], xv[NS], dv[NS], yv[NS], d0[NS], d1[NS];
+    int64_t eb[NS];  // first entry of the slice, or of the row
+#pragma unroll
+    for (int u = 0; u < NS; u++) {
+        const int row0 = (s0 + u) * RW;
+        bv[u] = xv[u] = dv[u] = yv[u] = d0[u] = d1[u] = 0;
+        eb[u] = (int64_t)row0 * NF;
+        if (orow && row0 + (int)r < nbr) {  // nbr: rows of this part
+            if constexpr (MAP) eb[u] = (int64_t)rowmap[row0 + r] * NF;
+            if (MODE != OP_SPMV) bv[u] = (AT)(b + eb[u])[eo];
+            if (SMOOTHING) xv[u] = (AT)(x + eb[u])[eo];
+            if (MODE == OP_CHEB && alpha != 0.0) dv[u] = (AT)(aux + eb[u])[eo];
+            if (MODE == OP_SPMV && beta != 0.0) yv[u] = (AT)(y + eb[u])[eo];
+        }
+        if (dlane && row0 + (int)dr < nbr) {
+            const TD* D = invD + (int64_t)(MAP ? rowmap[row0 + dr] : row0) * (NF * NF);
+            d0[u] = (AT)ldv(D + doff);
+            if constexpr (CW == 2) d1[u] = (AT)ldv(D + doff + 1);
+        }
+    }
+    // x of padding slots is taken as zero without a load
+    TV x0[NS], x1[NS];
+#pragma unroll
+    for (int u = 0; u < NS; u++) {
+        x0[u] = x1[u] = 0;
+        if constexpr (CW == 2) {
+            if (c[u] >= 0) ld2(x + (int64_t)c[u] * NF + 2 * jp, x0[u], x1[u]);
+        } else {
+            if (c[u] >= 0) x0[u] = x[(int64_t)c[u] * NF + jp];
+        }
     }
 
-    AT acc[NF];
 #pragma unroll
-    for (int k = 0; k < NF; k++) acc[k] = 0;
-    if (act) {
-        // x of padding slots is taken as zero without a load
-        if constexpr (CW == 2) {
-            TV x0 = 0, x1 = 0;
-            if (c >= 0) ld2(x + (int64_t)c * NF + 2 * jp, x0, x1);
+    for (int u = 0; u < NS; u++) {
+        if (u > 0 && s0 + u >= nslices) return;  // wavefront-uniform
+        const bool out = orow && (s0 + u) * RW + (int)r < nbr;
+        // Row k of the wavefront's LDS holds the 64 partial sums of entry k;
+        // the pitch keeps lanes that sum different entries in different banks.
+        if (u > 0) wave_lds_sync();  // the rows of the slice before have been read
+        AT* rw = red[wave];
 #pragma unroll
-            for (int k = 0; k < NF; k++) acc[k] = (AT)a[k][0] * (AT)x0 + (AT)a[k][1] * (AT)x1;
-        } else {
-            const AT x0 = c >= 0 ? (AT)x[(int64_t)c * NF + jp] : (AT)0;
-#pragma unroll
-            for (int k = 0; k < NF; k++) acc[k] = (AT)a[k][0] * x0;
-        }
-    }
-    // Row k of the wavefront's LDS holds the 64 partial sums of entry k,
-    // rotated by k so that the lanes summing different entries read
-    // different banks.
-#pragma unroll
-    for (int k = 0; k < NF; k++) red[wave][k][(lane + k) & 63] = acc[k];
-    wave_lds_sync();
-    // Row sums: NP lanes per (row r, entry i) each add a run of the LPR
-    // partial sums, then a shuffle tree over the parts leaves the row sum in
-    // part 0 (the other parts end with partial or foreign sums, not used).
-    const int QC = (LPR + NP - 1) / NP;
-    AT sum = 0;
-    if (r < RW) {
-        const int q1 = min(LPR, (part + 1) * QC);
-        for (int q = part * QC; q < q1; q++) sum += red[wave][i][(r * LPR + q + i) & 63];
-    }
-    for (int off = NP >> 1; off > 0; off >>= 1) sum += __shfl(sum, min(lane + NF * off, 63), 64);
-    if (MODE == OP_SPMV) {
-        if (out) {
-            AT v = (AT)alpha * sum;
-            if (beta != 0.0) v += (AT)beta * yv;
-            y[e] = (TV)v;
-        }
-    } else if (MODE == OP_RESID) {
-        if (out) y[e] = (TV)(bv - sum);
-    } else {
-        // z = D^-1 (b - A x) of the row's NF residuals
-        const AT res = bv - sum;
-        AT z = 0;
-        if (dist) {
-            const int src = min(dr * NF * NP + CW * dm, 63);
-            AT zp = __shfl(res, src, 64) * d0;
-            if constexpr (CW == 2) zp += __shfl(res, min(src + 1, 63), 64) * d1;
-            z = zp;
-            for (int p = 1; p < JP; p++) {
-                const AT o = __shfl(zp, min(lane + p, 63), 64);
-                if (dm == 0) z += o;
+        for (int k = 0; k < NF; k++) {
+            AT acc = 0;
+            if (act) {
+                if constexpr (CW == 2)
+                    acc = (AT)a[u][k].get(0) * (AT)x0[u] + (AT)a[u][k].get(1) * (AT)x1[u];
+                else
+                    acc = (AT)a[u][k].get(0) * (AT)x0[u];
             }
-            z = __shfl(z, min(r * NF * JP + i * JP, 63), 64);
-        } else {
-            // the residuals go through the wavefront's LDS rows, whose
-            // partial sums have all been read
-            AT* rs = &red[wave][0][0];
-            wave_lds_sync();
-            if (out) rs[r * NF + i] = res;
-            wave_lds_sync();
+            rw[k * kRedPitch + lane] = acc;
+        }
+        wave_lds_sync();
+        // Row sums: NP lanes per (row r, entry i) each add a run of the LPR
+        // partial sums, then a shuffle tree over the parts leaves the row sum in
+        // part 0 (the other parts end with partial or foreign sums, not used).
+        const int QC = (LPR + (1 << lognp) - 1) >> lognp;
+        AT sum = 0;
+        if (r < (unsigned)RW) {
+            const int n = min(LPR - (int)__umul24(part, QC), QC), full = LPR - ((1 << lognp) - 1) * QC;
+            const AT* q = rw + __umul24(i, kRedPitch) + __umul24(r, LPR) + __umul24(part, QC);
+            int j = 0;
+            for (; j + kRedBatch <= full; j += kRedBatch) {  // every part has these
+                AT v[kRedBatch];
+#pragma unroll
+                for (int w = 0; w < kRedBatch; w++) v[w] = q[j + w];
+#pragma unroll
+                for (int w = 0; w < kRedBatch; w++) sum += v[w];
+            }
+            for (; j < QC; j += kRedBatch / 2) {
+                AT v[kRedBatch / 2];
+#pragma unroll
+                for (int w = 0; w < kRedBatch / 2; w++) v[w] = q[j + w];
+#pragma unroll
+                for (int w = 0; w < kRedBatch / 2; w++)
+                    if (j + w < n) sum += v[w];
+            }
+        }
+        for (int l = lognp - 1; l >= 0; l--) sum += __shfl(sum, min((int)lane + (NF << l), 63), 64);
+        if (MODE == OP_SPMV) {
             if (out) {
-                const TD* D = invD + e * NF;
-#pragma unroll
-                for (int k = 0; k < NF; k++) z += (AT)ldv(D + k) * rs[r * NF + k];
+                AT v = (AT)alpha * sum;
+                if (beta != 0.0) v += (AT)beta * yv[u];
+                (y + eb[u])[eo] = (TV)v;
             }
-        }
-        if (out) {
-            if constexpr (MODE == OP_CHEB) {
-                const AT dn = (alpha != 0.0 ? (AT)alpha * dv : (AT)0) + (AT)beta * z;
-                aux[e] = (TV)dn;
-                y[e] = (TV)(xv + dn);
+        } else if (MODE == OP_RESID) {
+            if (out) (y + eb[u])[eo] = (TV)(bv[u] - sum);
+        } else {
+            // z = D^-1 (b - A x) of the row's NF residuals
+            const AT res = bv[u] - sum;
+            AT z = 0;
+            if (dist) {
+                const int src = min((int)(((dr * NF) << lognp) + CW * dm), 63);
+                AT zp = __shfl(res, src, 64) * d0[u];
+                if constexpr (CW == 2) zp += __shfl(res, min(src + 1, 63), 64) * d1[u];
+                z = zp;
+                for (int p = 1; p < JP; p++) {
+                    const AT o = __shfl(zp, min((int)lane + p, 63), 64);
+                    if (dm == 0) z += o;
+                }
+                z = __shfl(z, min((int)((r * NF + i) * JP), 63), 64);
             } else {
-                y[e] = (TV)(xv + (AT)omega * z);
+                // the residuals go through the wavefront's LDS rows, whose
+                // partial sums have all been read
+                wave_lds_sync();
+                if (out) rw[r * NF + i] = res;
+                wave_lds_sync();
+                if (out) {
+                    const TD* D = invD + (eb[u] + eo) * NF;
+#pragma unroll
+                    for (int k = 0; k < NF; k++) z += (AT)ldv(D + k) * rw[r * NF + k];
+                }
+            }
+            if (out) {
+                if constexpr (MODE == OP_CHEB) {
+                    const AT dn = (alpha != 0.0 ? (AT)alpha * dv[u] : (AT)0) + (AT)beta * z;
+                    (aux + eb[u])[eo] = (TV)dn;
+                    (y + eb[u])[eo] = (TV)(xv[u] + dn);
+                } else {
+                    (y + eb[u])[eo] = (TV)(xv[u] + (AT)omega * z);
+                }
             }
         }
     }
@@ -1235,6 +1289,21 @@ int bcsr_variant() {
     return v;
 }
 
+// log2 of the lanes that add the sums of one (row, entry) of a slice
+int sliced_lognp(int entries) {
+    int l = 0;
+    while (entries << (l + 1) <= 64) l++;
+    return l;
+}
+
+// Slices per wavefront of the sliced kernels: two share the index arithmetic
+// and have twice the loads in flight, but halve the number of wavefronts.
+// From 64 wavefronts per CU on two are the faster (47 600 slices of n_f = 6 in
+// BF16: 34.1 us a call, 37.8 us with one; 60 000 of n_f = 3 in FP32: 32.0 and
+// 36.5 us), below one (22 800 smoothing slices of n_f = 6 in FP64: 53 us a
+// call, 58 us with two).
+int slices_per_wave(int nslices) { return nslices >= 2 * 64 * 256 ? 2 : 1; }
+
 template <int NF, class TA, class TV, class TD>
 void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, const void* b, void* y, double alpha,
                         double beta, double omega, const void* invD, const int* rows, int nrows, void* aux) {
@@ -1315,17 +1384,24 @@ void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, con
             auto sv = S.vals.as<TA>();
             auto rm = S.rowmap.as<int>();
             const int nrp = S.nrows;
-            auto kern = rm ? (mode == OP_SPMV    ? k_sliced<NF, TA, TV, TD, OP_SPMV, true>
-                              : mode == OP_RESID ? k_sliced<NF, TA, TV, TD, OP_RESID, true>
-                              : mode == OP_CHEB  ? k_sliced<NF, TA, TV, TD, OP_CHEB, true>
-                                                 : k_sliced<NF, TA, TV, TD, OP_SMOOTH, true>)
-                           : (mode == OP_SPMV    ? k_sliced<NF, TA, TV, TD, OP_SPMV, false>
-                              : mode == OP_RESID ? k_sliced<NF, TA, TV, TD, OP_RESID, false>
-                              : mode == OP_CHEB  ? k_sliced<NF, TA, TV, TD, OP_CHEB, false>
-                                                 : k_sliced<NF, TA, TV, TD, OP_SMOOTH, false>);
-            const int nwg = (S.nslices + kSlicedWaves - 1) / kSlicedWaves;
-            hipLaunchKernelGGL(kern, dim3(nwg), dim3(kWG), 0, c.stream, nrp, S.nslices, S.W, S.RW, sc, sv, xx, bb, yy,
-                               alpha, beta, omega, D, ax, rm);
+            constexpr int JP = NF % 2 == 0 ? NF / 2 : NF;
+            const int ns = slices_per_wave(S.nslices);
+            auto pick = [&](auto nst) {
+                constexpr int NS = decltype(nst)::value;
+                return rm ? (mode == OP_SPMV    ? k_sliced<NF, TA, TV, TD, OP_SPMV, true, NS>
+                             : mode == OP_RESID ? k_sliced<NF, TA, TV, TD, OP_RESID, true, NS>
+                             : mode == OP_CHEB  ? k_sliced<NF, TA, TV, TD, OP_CHEB, true, NS>
+                                                : k_sliced<NF, TA, TV, TD, OP_SMOOTH, true, NS>)
+                          : (mode == OP_SPMV    ? k_sliced<NF, TA, TV, TD, OP_SPMV, false, NS>
+                             : mode == OP_RESID ? k_sliced<NF, TA, TV, TD, OP_RESID, false, NS>
+                             : mode == OP_CHEB  ? k_sliced<NF, TA, TV, TD, OP_CHEB, false, NS>
+                                                : k_sliced<NF, TA, TV, TD, OP_SMOOTH, false, NS>);
+            };
+            auto kern = ns == 2 ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 1>{});
+            const int nwg = (S.nslices + kSlicedWaves * ns - 1) / (kSlicedWaves * ns);
+            hipLaunchKernelGGL(kern, dim3(nwg), dim3(kWG), 0, c.stream, nrp, S.nslices, S.W, S.RW,
+                               (int)small_rcp(S.W * JP), sliced_lognp(S.RW * NF), sc, sv, xx, bb, yy, alpha, beta,
+                               omega, D, ax, rm);
             FH_HIP(hipGetLastError());
         }
         return;
@@ -1859,8 +1935,9 @@ static bool spmv_f32vals_nf(Ctx& c, const Bcsr& A, const void* x, void* y) {
         if (S.kind != 0 || S.next || S.rowmap.p) return false;
         if (S.cw == 2 && (uintptr_t)x % 16 != 0) return false;
         const int nwg = (S.nslices + kSlicedWaves - 1) / kSlicedWaves;
-        hipLaunchKernelGGL((k_sliced<NF, float, double, double, OP_SPMV, false>), dim3(nwg), dim3(kWG), 0, c.stream,
-                           S.nrows, S.nslices, S.W, S.RW, S.cols.as<int>(), S.vals.as<float>(), (const double*)x,
+        hipLaunchKernelGGL((k_sliced<NF, float, double, double, OP_SPMV, false, 1>), dim3(nwg), dim3(kWG), 0, c.stream,
+                           S.nrows, S.nslices, S.W, S.RW, (int)small_rcp(S.W * (NF % 2 == 0 ? NF / 2 : NF)),
+                           sliced_lognp(S.RW * NF), S.cols.as<int>(), S.vals.as<float>(), (const double*)x,
                            (const double*)nullptr, (double*)y, 1.0, 0.0, 0.0, (const double*)nullptr,
                            (double*)nullptr, (const int*)nullptr);
     }
