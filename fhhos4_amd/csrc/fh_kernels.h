@@ -10,6 +10,8 @@ enum BcsrMode : int {
     OP_RESID = 1,   // y = b - A x
     OP_SMOOTH = 2,  // y = x + omega * D^-1 (b - A x)   (block Jacobi / GS colour)
     OP_CHEB = 3,    // d = alpha * d + beta * D^-1 (b - A x), y = x + d   (Chebyshev step)
+    OP_CHEB_ZERO = 5,     // OP_CHEB from x = d = omega D^-1 b, scalar rows (launch_cheb_start)
+    OP_CHEB_PROLONG = 6,  // OP_CHEB from x + ec[agg], scalar rows (launch_cheb_start)
     OP_RESID_HEAD = 4,  // rc[i] = (b - A x)[i nf]: launch_resid_head (in-situ timing code only)
 };
 
@@ -25,6 +27,15 @@ void launch_bcsr(Ctx& c, const Bcsr& A, BcsrMode mode, Prec vprec, const void* x
 // (d not read when a = 0) and xnew = x + d.  xnew must not alias x.
 void launch_bcsr_cheb(Ctx& c, const Bcsr& A, Prec vprec, const void* x, const void* b, void* xnew, void* d,
                       double a, double cc, const void* invD, Prec dprec);
+
+// A Chebyshev step on scalar rows that forms the vector it starts from while it
+// reads it: omega D^-1 b, also the direction (agg null; the second step from
+// zero, x is not read), or x + ec[agg] (the step after an aggregation
+// prolongation; x stays as it is).  Returns false, having launched nothing,
+// where the two passes are as fast and while launches are timed.
+bool launch_cheb_start(Ctx& c, const Bcsr& A, Prec vprec, const void* x, const void* b, void* xnew, void* d,
+                       double omega, const int* agg, const void* ec, double a, double cc, const void* invD,
+                       Prec dprec);
 
 // rc[i] = (b - A x)[i nf] for every block row i: the residual truncated to
 // the first mode of each block (the p-restriction to one mode per face),

@@ -134,6 +134,27 @@ __global__ __launch_bounds__(kWG) void k_bcsr(int nbr, const int* __restrict__ r
     }
 }
 
+// Entry j of the vector that a Chebyshev step on scalar rows starts from:
+//   OP_CHEB          x
+//   OP_CHEB_ZERO     omega D^-1 b, the first step from zero (k_bjac_zero)
+//   OP_CHEB_PROLONG  x + ec[agg], the coarse correction (k_agg_prolong_add)
+// formed where it is read: one entry more per stored entry of A, but a launch
+// and a pass less.  Rounded like the stored vectors.
+template <int MODE, class TV, class TD>
+__device__ __forceinline__ TV start_entry(int64_t j, const TV* x, const TV* b, const TD* __restrict__ invD,
+                                          double omega, const int* __restrict__ agg, const TV* __restrict__ ec) {
+#pragma clang fp contract(off)
+    using AT = typename Acc<TV>::T;
+    if constexpr (MODE == OP_CHEB_ZERO) {
+        const AT z = (AT)ldv(invD + j) * (AT)b[j];
+        return (TV)((AT)omega * z);
+    } else if constexpr (MODE == OP_CHEB_PROLONG) {
+        return (TV)((AT)x[j] + (AT)ec[agg[j]]);
+    } else {
+        return x[j];
+    }
+}
+
 // Scalar rows (n_f = 1): a group of G lanes per row (64 / G rows per
 // wavefront), the lanes of a group striding over the row's entries, the
 // partial sums reduced with xor-shuffles inside the group.  For the
@@ -144,7 +165,8 @@ __global__ __launch_bounds__(kWG) void k_csr_grp(int nbr, const int* __restrict_
                                                   const TA* __restrict__ val, const TV* x, const TV* __restrict__ b,
                                                   TV* y, double alpha, double beta, double omega,
                                                   const TD* __restrict__ invD, const int* __restrict__ rows,
-                                                  int nrows, TV* __restrict__ aux) {
+                                                  int nrows, TV* __restrict__ aux, const int* __restrict__ agg,
+                                                  const TV* __restrict__ ec) {
     using AT = typename Acc<TV>::T;
     const int lane = threadIdx.x & 63;
     const int wg = xcd_remap(blockIdx.x, gridDim.x);
@@ -158,7 +180,8 @@ __global__ __launch_bounds__(kWG) void k_csr_grp(int nbr, const int* __restrict_
     if (idx < count) {
         br = rows ? rows[idx] : idx;
         const int s = rp[br], e = rp[br + 1];
-        for (int p = s + gl; p < e; p += G) acc += (AT)ldv(val + p) * (AT)x[ci[p]];
+        for (int p = s + gl; p < e; p += G)
+            acc += (AT)ldv(val + p) * (AT)start_entry<MODE>(ci[p], x, b, invD, omega, agg, ec);
     }
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
@@ -172,7 +195,15 @@ __global__ __launch_bounds__(kWG) void k_csr_grp(int nbr, const int* __restrict_
         y[row] = (TV)((AT)b[row] - acc);
     } else {
         const AT z = (AT)ldv(invD + row) * ((AT)b[row] - acc);
-        smooth_out<MODE>(row, z, x, y, aux, alpha, beta, omega);
+        if constexpr (MODE == OP_CHEB_ZERO || MODE == OP_CHEB_PROLONG) {
+            const AT xv = (AT)start_entry<MODE>(row, x, b, invD, omega, agg, ec);
+            const AT dv = MODE == OP_CHEB_ZERO ? xv : (alpha != 0.0 ? (AT)aux[row] : (AT)0);
+            const AT dn = (alpha != 0.0 ? (AT)alpha * dv : (AT)0) + (AT)beta * z;
+            aux[row] = (TV)dn;
+            y[row] = (TV)(xv + dn);
+        } else {
+            smooth_out<MODE>(row, z, x, y, aux, alpha, beta, omega);
+        }
     }
 }
 
@@ -833,8 +864,12 @@ __global__ __launch_bounds__(kWG) void k_sell(int nbr, int nslices, const int* _
     const bool out = row < nbr;
     if (out) {
         if (MODE != OP_SPMV) bv = (AT)b[row];
-        if (MODE == OP_CHEB || MODE == OP_SMOOTH) { xv = (AT)x[row]; dinv = (AT)ldv(invD + row); }
-        if (MODE == OP_CHEB && alpha != 0.0) dv = (AT)aux[row];
+        if (MODE != OP_SPMV && MODE != OP_RESID) {
+            xv = (AT)start_entry<MODE>(row, x, b, invD, omega, nullptr, (const TV*)nullptr);
+            dinv = (AT)ldv(invD + row);
+        }
+        if (MODE == OP_CHEB_ZERO) dv = xv;
+        else if (MODE == OP_CHEB && alpha != 0.0) dv = (AT)aux[row];
         if (MODE == OP_SPMV && beta != 0.0) yv = (AT)y[row];
     }
     // batches of kSellBatch slots (beyond w: the last one again, not added)
@@ -853,7 +888,7 @@ __global__ __launch_bounds__(kWG) void k_sell(int nbr, int nslices, const int* _
         LT ac[kSellBatch];
 #pragma unroll
         for (int u = 0; u < kSellBatch; u++) {
-            xc[u] = (AT)x[c[u]];
+            xc[u] = (AT)start_entry<MODE>(c[u], x, b, invD, omega, nullptr, (const TV*)nullptr);
             ac[u] = a[u];
         }
         if (j + kSellBatch < w) load(j + kSellBatch);
@@ -868,7 +903,7 @@ __global__ __launch_bounds__(kWG) void k_sell(int nbr, int nslices, const int* _
         y[row] = (TV)v;
     } else if constexpr (MODE == OP_RESID) {
         y[row] = (TV)(bv - acc);
-    } else if constexpr (MODE == OP_CHEB) {
+    } else if constexpr (MODE != OP_SMOOTH) {  // Chebyshev step
         const AT dn = (alpha != 0.0 ? (AT)alpha * dv : (AT)0) + (AT)beta * dinv * (bv - acc);
         aux[row] = (TV)dn;
         y[row] = (TV)(xv + dn);
@@ -1264,7 +1299,19 @@ __global__ __launch_bounds__(kWG) void k_dense_symv(int n, const TM* __restrict_
     if (row >= n) return;
     const TM* m = M + (int64_t)row * n;
     AT s = 0;
-    for (int j = lane; j < n; j += 64) s += (AT)ldv(m + j) * (AT)x[j];
+    int j = lane;
+    for (; j + 7 * 64 < n; j += 8 * 64) {  // eight loads in flight, added in order
+        TM a[8];
+        TV v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            a[u] = m[j + 64 * u];
+            v[u] = x[j + 64 * u];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) s += (AT)ldv(a + u) * (AT)v[u];
+    }
+    for (; j < n; j += 64) s += (AT)ldv(m + j) * (AT)x[j];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
     if (lane == 0) y[row] = (TV)s;
@@ -1306,7 +1353,8 @@ int slices_per_wave(int nslices) { return nslices >= 2 * 64 * 256 ? 2 : 1; }
 
 template <int NF, class TA, class TV, class TD>
 void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, const void* b, void* y, double alpha,
-                        double beta, double omega, const void* invD, const int* rows, int nrows, void* aux) {
+                        double beta, double omega, const void* invD, const int* rows, int nrows, void* aux,
+                        const int* agg, const void* ecv) {
     int count = rows ? nrows : A.nbr;
     if (count <= 0) return;
     auto rp = A.rowptr.as<int>();
@@ -1317,6 +1365,7 @@ void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, con
     auto yy = (TV*)y;
     auto D = (const TD*)invD;
     auto ax = (TV*)aux;
+    auto ec = (const TV*)ecv;
     if constexpr (NF == 1) {
         if (!rows && A.sliced_state == 1 && A.sliced->kind == 2) {
             const Sliced& S = *A.sliced;
@@ -1335,6 +1384,10 @@ void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, con
                     break;
                 case OP_CHEB:
                     hipLaunchKernelGGL((k_sell<TA, TV, TD, OP_CHEB>), dim3(nwg), dim3(kWG), 0, c.stream, A.nbr,
+                                       S.nslices, sp, sc, sv, xx, bb, yy, alpha, beta, omega, D, ax);
+                    break;
+                case OP_CHEB_ZERO:
+                    hipLaunchKernelGGL((k_sell<TA, TV, TD, OP_CHEB_ZERO>), dim3(nwg), dim3(kWG), 0, c.stream, A.nbr,
                                        S.nslices, sp, sc, sv, xx, bb, yy, alpha, beta, omega, D, ax);
                     break;
                 default:
@@ -1439,7 +1492,7 @@ void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, con
         const int nwg = (int)(((int64_t)count * G + kWG - 1) / kWG);
 #define FH_CSR(GG, MD)                                                                                              \
         hipLaunchKernelGGL((k_csr_grp<GG, TA, TV, TD, MD>), dim3(nwg), dim3(kWG), 0, c.stream, A.nbr, rp, ci, val, \
-                           xx, bb, yy, alpha, beta, omega, D, rows, nrows, ax)
+                           xx, bb, yy, alpha, beta, omega, D, rows, nrows, ax, agg, ec)
 #define FH_CSR_G(MD)                          \
         switch (G) {                           \
             case 4: FH_CSR(4, MD); break;      \
@@ -1451,6 +1504,8 @@ void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, con
             case OP_SPMV: FH_CSR_G(OP_SPMV); break;
             case OP_RESID: FH_CSR_G(OP_RESID); break;
             case OP_CHEB: FH_CSR_G(OP_CHEB); break;
+            case OP_CHEB_ZERO: FH_CSR_G(OP_CHEB_ZERO); break;
+            case OP_CHEB_PROLONG: FH_CSR_G(OP_CHEB_PROLONG); break;
             default: FH_CSR_G(OP_SMOOTH); break;
         }
 #undef FH_CSR_G
@@ -1483,17 +1538,21 @@ void bcsr_dispatch_mode(Ctx& c, const Bcsr& A, BcsrMode mode, const void* x, con
 template <int NF>
 void bcsr_dispatch_types(Ctx& c, const Bcsr& A, BcsrMode mode, Prec vp, const void* x, const void* b, void* y,
                          double alpha, double beta, double omega, const void* invD, Prec dp, const int* rows,
-                         int nrows, void* aux) {
+                         int nrows, void* aux, const int* agg, const void* ec) {
+    const bool inv = mode != OP_SPMV && mode != OP_RESID;
     if (vp == Prec::F64) {
-        FH_CHECK(A.prec == Prec::F64 && ((mode != OP_SMOOTH && mode != OP_CHEB) || dp == Prec::F64), -3,
+        FH_CHECK(A.prec == Prec::F64 && (!inv || dp == Prec::F64), -3,
                  "FP64 vectors need FP64 matrix and FP64 block inverses");
-        bcsr_dispatch_mode<NF, double, double, double>(c, A, mode, x, b, y, alpha, beta, omega, invD, rows, nrows, aux);
+        bcsr_dispatch_mode<NF, double, double, double>(c, A, mode, x, b, y, alpha, beta, omega, invD, rows, nrows, aux,
+                                                 agg, ec);
     } else if (vp == Prec::F32) {
-        FH_CHECK((mode != OP_SMOOTH && mode != OP_CHEB) || dp == Prec::F32, -3, "FP32 smoothing needs FP32 block inverses");
+        FH_CHECK(!inv || dp == Prec::F32, -3, "FP32 smoothing needs FP32 block inverses");
         if (A.prec == Prec::F32)
-            bcsr_dispatch_mode<NF, float, float, float>(c, A, mode, x, b, y, alpha, beta, omega, invD, rows, nrows, aux);
+            bcsr_dispatch_mode<NF, float, float, float>(c, A, mode, x, b, y, alpha, beta, omega, invD, rows, nrows, aux,
+                                                 agg, ec);
         else if (A.prec == Prec::BF16)
-            bcsr_dispatch_mode<NF, bf16_t, float, float>(c, A, mode, x, b, y, alpha, beta, omega, invD, rows, nrows, aux);
+            bcsr_dispatch_mode<NF, bf16_t, float, float>(c, A, mode, x, b, y, alpha, beta, omega, invD, rows, nrows, aux,
+                                                 agg, ec);
         else
             throw Error(-3, "FP32 vectors need an FP32 or BF16 matrix");
     } else
@@ -1871,7 +1930,7 @@ void* noalloc_scratch(int device) {
 
 static void launch_bcsr_impl(Ctx& c, const Bcsr& A, BcsrMode mode, Prec vprec, const void* x, const void* b, void* y,
                              double alpha, double beta, double omega, const void* invD, Prec dprec, const int* rows,
-                             int nrows, void* aux);
+                             int nrows, void* aux, const int* agg = nullptr, const void* ec = nullptr);
 
 void launch_bcsr(Ctx& c, const Bcsr& A, BcsrMode mode, Prec vprec, const void* x, const void* b, void* y,
                  double alpha, double beta, double omega, const void* invD, Prec dprec, const int* rows,
@@ -1917,6 +1976,25 @@ void launch_bcsr_cheb(Ctx& c, const Bcsr& A, Prec vprec, const void* x, const vo
         FH_HIP(hipEventRecord(e1, c.stream));
         c.prof_events.push_back({e0, e1});
     }
+}
+
+bool launch_cheb_start(Ctx& c, const Bcsr& A, Prec vprec, const void* x, const void* b, void* xnew, void* d,
+                       double omega, const int* agg, const void* ec, double a, double cc, const void* invD,
+                       Prec dprec) {
+    if (A.bs_r != 1 || A.bs_c != 1 || A.elem_on || c.prof_matrix == (const void*)&A) return false;
+    if (A.sliced_state == 0 && !c.no_alloc) sliced_decide(c, A);
+    // The correction on SELL-64 levels stays a pass of its own: 26 167 rows
+    // (FP64) take 8.4 us fused and 5.3 + 3.2 us apart, 95 232 rows 10.0 us and
+    // 6.2 + 3.1 us; 7 663 rows in CSR take 4.6 us and 3.4 + 3.0 us.  The start
+    // from zero takes 7.8 us for 6.2 + 4.6 us at 95 232 rows, 7.2 us for
+    // 6.4 + 4.0 us at 61 851 (FP32), but 14.4 us for 9.7 + 4.5 us at 212 117.
+    if (!agg && A.nbr > 131072) return false;
+    if (A.sliced_state == 1 && (A.sliced->kind != 2 || agg)) return false;
+    FH_CHECK(xnew != x && xnew != b && d != nullptr && d != x && d != xnew, -3,
+             "Chebyshev step: x, xnew and d must differ");
+    launch_bcsr_impl(c, A, agg ? OP_CHEB_PROLONG : OP_CHEB_ZERO, vprec, x, b, xnew, a, cc, omega, invD, dprec, nullptr,
+                     0, d, agg, ec);
+    return true;
 }
 
 // y = A x with FP32-stored values and FP64 vectors (FP64 accumulation), on
@@ -2037,15 +2115,15 @@ bool launch_resid_head(Ctx& c, const Bcsr& A, Prec vp, const void* x, const void
 
 static void launch_bcsr_impl(Ctx& c, const Bcsr& A, BcsrMode mode, Prec vprec, const void* x, const void* b, void* y,
                              double alpha, double beta, double omega, const void* invD, Prec dprec, const int* rows,
-                             int nrows, void* aux) {
+                             int nrows, void* aux, const int* agg, const void* ec) {
     FH_CHECK(A.bs_r == A.bs_c, -3, "block-row kernel needs square blocks");
     switch (A.bs_r) {
-        case 1: bcsr_dispatch_types<1>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux); break;
-        case 2: bcsr_dispatch_types<2>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux); break;
-        case 3: bcsr_dispatch_types<3>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux); break;
-        case 4: bcsr_dispatch_types<4>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux); break;
-        case 6: bcsr_dispatch_types<6>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux); break;
-        case 10: bcsr_dispatch_types<10>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux); break;
+        case 1: bcsr_dispatch_types<1>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux, agg, ec); break;
+        case 2: bcsr_dispatch_types<2>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux, agg, ec); break;
+        case 3: bcsr_dispatch_types<3>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux, agg, ec); break;
+        case 4: bcsr_dispatch_types<4>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux, agg, ec); break;
+        case 6: bcsr_dispatch_types<6>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux, agg, ec); break;
+        case 10: bcsr_dispatch_types<10>(c, A, mode, vprec, x, b, y, alpha, beta, omega, invD, dprec, rows, nrows, aux, agg, ec); break;
         default: throw Error(-3, "unsupported block size " + std::to_string(A.bs_r) + " (1,2,3,4,6,10)");
     }
 }

@@ -268,8 +268,12 @@ static void gs_sweep(Ctx& c, const Bcsr& A, LevelSmoother& S, Prec vp, const voi
 }
 
 void smoother_apply(Ctx& c, const Bcsr& A, LevelSmoother& S, Prec vp, const void* b, DVec& x, DVec& work,
-                    bool& x_is_zero) {
+                    bool& x_is_zero, const int* agg, const void* ec) {
     const int nf = A.bs_r;
+    if (agg && (S.spec.kind != SmootherKind::Chebyshev || S.spec.iterations == 0 || nf != 1)) {
+        launch_agg_prolong_add(c, A.nbr, nf, vp, agg, ec, x.data());
+        agg = nullptr;
+    }
     for (int it = 0; it < S.spec.iterations; it++) {
         if (S.spec.kind == SmootherKind::BlockJacobi) {
             if (x_is_zero)
@@ -284,11 +288,15 @@ void smoother_apply(Ctx& c, const Bcsr& A, LevelSmoother& S, Prec vp, const void
             const double hi = kChebHigh * S.lmax, lo = kChebLow * S.lmax;
             const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
             double rho = 1.0 / sigma;
+            bool at_start = false;  // x = d = D^-1 b / theta, not formed yet
             for (int k = 0; k < S.spec.degree; k++) {
                 if (k == 0 && x_is_zero) {
-                    // from x = 0: d = D^-1 b / theta and x = d in one pass
-                    launch_bjac_zero(c, A.nbr, nf, vp, b, x.data(), 1.0 / theta, S.invD->p, S.dprec, nullptr, 0,
-                                     S.d.data());
+                    // from x = 0: d = D^-1 b / theta and x = d in one pass, or
+                    // within the next step on scalar rows
+                    at_start = S.spec.degree > 1 && nf == 1;
+                    if (!at_start)
+                        launch_bjac_zero(c, A.nbr, nf, vp, b, x.data(), 1.0 / theta, S.invD->p, S.dprec, nullptr, 0,
+                                         S.d.data());
                 } else {
                     // d = a d + c D^-1 (b - A x) and x + d in one block-row pass
                     // into work, which then becomes x
@@ -299,7 +307,19 @@ void smoother_apply(Ctx& c, const Bcsr& A, LevelSmoother& S, Prec vp, const void
                         cc = 2.0 * rn / delta;
                         rho = rn;
                     }
-                    launch_bcsr_cheb(c, A, vp, x.data(), b, work.data(), S.d.data(), a, cc, S.invD->p, S.dprec);
+                    bool done = false;
+                    if (at_start || agg) {
+                        done = launch_cheb_start(c, A, vp, x.data(), b, work.data(), S.d.data(), 1.0 / theta,
+                                                 at_start ? nullptr : agg, ec, a, cc, S.invD->p, S.dprec);
+                        if (!done && at_start)
+                            launch_bjac_zero(c, A.nbr, nf, vp, b, x.data(), 1.0 / theta, S.invD->p, S.dprec, nullptr,
+                                             0, S.d.data());
+                        else if (!done)
+                            launch_agg_prolong_add(c, A.nbr, nf, vp, agg, ec, x.data());
+                        at_start = false;
+                        agg = nullptr;
+                    }
+                    if (!done) launch_bcsr_cheb(c, A, vp, x.data(), b, work.data(), S.d.data(), a, cc, S.invD->p, S.dprec);
                     std::swap(x.buf, work.buf);
                 }
                 x_is_zero = false;
@@ -635,8 +655,6 @@ private:
         MgLevel& V = L[l];
         if (V.ptrunc)
             launch_p_prolong_add(c_, V.A64->nbr, V.A64->bs_r, V.nfc, vp_, ec.data(), x.data());
-        else if (V.agg)
-            launch_agg_prolong_add(c_, V.A64->nbr, V.A64->bs_r, vp_, V.agg_map.as<int>(), ec.data(), x.data());
         else
             launch_bcsr(c_, *V.Pw, OP_SPMV, vp_, ec.data(), nullptr, x.data(), 1.0, 1.0, 0.0, nullptr, vp_, nullptr, 0);
     }
@@ -673,8 +691,12 @@ public:
             }
         }
         if (xz) { launch_fill(c_, V.n, x.data(), vp_, 0.0); xz = false; }
-        prolong_add(l, C.x, x);
-        smoother_apply(c_, *V.Aw, V.post, vp_, b, x, V.work, xz);
+        if (V.agg) {
+            smoother_apply(c_, *V.Aw, V.post, vp_, b, x, V.work, xz, V.agg_map.as<int>(), C.x.data());
+        } else {
+            prolong_add(l, C.x, x);
+            smoother_apply(c_, *V.Aw, V.post, vp_, b, x, V.work, xz);
+        }
         if (Ax) launch_bcsr(c_, *V.Aw, OP_SPMV, vp_, x.data(), nullptr, Ax->data(), 1.0, 0.0, 0.0, nullptr, vp_, nullptr, 0);
     }
 

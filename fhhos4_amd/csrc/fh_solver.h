@@ -212,8 +212,9 @@ private:
 };
 
 // Smoother application on one level (in the level's working precision).
+// With agg the coarse correction ec is added to x first (x[i] += ec[agg[i]]).
 void smoother_setup(Ctx& c, const Bcsr& A64, LevelSmoother& S, Prec dprec);
 void smoother_apply(Ctx& c, const Bcsr& A, LevelSmoother& S, Prec vp, const void* b, DVec& x, DVec& work,
-                    bool& x_is_zero);
+                    bool& x_is_zero, const int* agg = nullptr, const void* ec = nullptr);
 
 }  // namespace fh
