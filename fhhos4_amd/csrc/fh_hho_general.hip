@@ -309,6 +309,7 @@ __global__ __launch_bounds__(NW * 64, MW) void k_hho_general(HhoDev d, int* err)
                 TabRef L[3], D[3];
                 refs(tab, L, D);
                 const double r0 = 1.0 / hw[0], r1 = 1.0 / hw[1], r2 = 1.0 / hw[2];
+#pragma unroll 2
                 for (int q = bq; q < ns * QS; q += NT / NR) {
                     const double L0 = L[0].at(q), L1 = L[1].at(q), L2 = DIM == 3 ? L[2].at(q) : 1.0;
                     const double D0 = D[0].at(q), D1 = D[1].at(q), D2 = DIM == 3 ? D[2].at(q) : 0.0;
@@ -326,6 +327,7 @@ __global__ __launch_bounds__(NW * 64, MW) void k_hho_general(HhoDev d, int* err)
 #pragma unroll
                     for (int j = 0; j < T; j++) s[i][j] = 0;
                 const double k0 = Kc[0], k1 = Kc[4], k2 = Kc[8];
+#pragma unroll 1
                 for (int q = ssl * QS; q < (ssl + 1) * QS; q++) {
                     const double* g = Gp + q * DIM * NR;
                     const double w = pt[2 * q];
@@ -493,6 +495,7 @@ __global__ __launch_bounds__(NW * 64, MW) void k_hho_general(HhoDev d, int* err)
             TabRef L[3], D[3];
             refs(sm + G::fTab, L, D);
             const double r0 = 1.0 / hw[0], r1 = 1.0 / hw[1], r2 = 1.0 / hw[2];
+#pragma unroll 2
             for (int q = bq; q < QF; q += NT / NR) {
                 const double L0 = L[0].at(q), L1 = L[1].at(q), L2 = DIM == 3 ? L[2].at(q) : 1.0;
                 const double D0 = D[0].at(q), D1 = D[1].at(q), D2 = DIM == 3 ? D[2].at(q) : 0.0;
@@ -931,7 +934,8 @@ void launch_hho_general(Ctx& c, const HhoDev& d) {
     // three to five to a SIMD: a few spilled registers cost less than the
     // latency that the other cells hide (12 167 hexahedra at k = 0: 109 us at
     // four, 121 us at three; k = 1: 317 us at three, 330 us at two, 354 us at
-    // four; 10 000 quadrilaterals at k = 3: 281 us at two, 301 us at three).
+    // four; 10 000 quadrilaterals at k = 3: 281 us at two, 301 us at three; 282
+    // and 249 us of the chosen ones since two points' tables are read at once).
     // At k = 2 and 3 in 3-D the tiles feed two and four wavefronts and the
     // factorisations need the registers of two per SIMD (k = 2: 1.11 ms with
     // two wavefronts, 1.67 ms with four; k = 3: 4.84 ms with four, 8.98 ms
