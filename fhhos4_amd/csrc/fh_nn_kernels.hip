@@ -35,8 +35,10 @@ __device__ __forceinline__ float wload(const bf16w* p) { return __uint_as_float(
 // v = D^-1 r1 (FP32) and the workgroup's share of |v|^2 (FP64), 256 / nf block
 // rows at a time: their inverse blocks (one contiguous span) and entries of r1
 // go through LDS, then thread t forms entry t of the tile.  Bound by reading
-// the inverse blocks; a thread per unknown that reads its row of D strided
-// took 21.5 us for 95 232 blocks of 10 x 10 (38 MB).
+// the inverse blocks: 12.6 us for 95 232 blocks of 10 x 10 (38 MB) with the next
+// tile's loads in flight, 25.5 us when a workgroup loads its tiles one after the
+// other (a thread per unknown that reads its row of D strided took 21.5 us,
+// without the norm).
 __global__ __launch_bounds__(256) void k_nn_prep(int n, int nf, const double* __restrict__ r1,
                                                  const float* __restrict__ invD, float* __restrict__ v,
                                                  double* __restrict__ partials) {
@@ -44,12 +46,27 @@ __global__ __launch_bounds__(256) void k_nn_prep(int n, int nf, const double* __
     __shared__ double sw[4];
     const int t = threadIdx.x, R = 256 / nf, b = t / nf;
     double vv = 0;
-    for (int64_t r0 = (int64_t)blockIdx.x * R; r0 < n; r0 += (int64_t)gridDim.x * R) {
-        const int rows = (int)min((int64_t)R, n - r0), nv = rows * nf, ne = nv * nf;
+    // the next tile's loads are in flight while this one is formed
+    float nd[kMaxNf];
+    double nr = 0;
+    auto fetch = [&](int64_t r0) {
+        const int nv = (int)min((int64_t)R, n - r0) * nf, ne = nv * nf;
         const float* D = invD + r0 * nf * nf;
-        for (int e = t; e < ne; e += 256) sD[e] = __builtin_nontemporal_load(D + e);
-        if (t < nv) sr[t] = (float)r1[r0 * nf + t];
+#pragma unroll
+        for (int u = 0; u < kMaxNf; u++)
+            if (t + 256 * u < ne) nd[u] = __builtin_nontemporal_load(D + t + 256 * u);
+        if (t < nv) nr = r1[r0 * nf + t];
+    };
+    const int64_t step = (int64_t)gridDim.x * R;
+    fetch((int64_t)blockIdx.x * R);  // every workgroup has a tile
+    for (int64_t r0 = (int64_t)blockIdx.x * R; r0 < n; r0 += step) {
+        const int nv = (int)min((int64_t)R, n - r0) * nf, ne = nv * nf;
+#pragma unroll
+        for (int u = 0; u < kMaxNf; u++)
+            if (t + 256 * u < ne) sD[t + 256 * u] = nd[u];
+        if (t < nv) sr[t] = (float)nr;
         __syncthreads();
+        if (r0 + step < n) fetch(r0 + step);
         if (t < nv) {
             float s = 0.f;
             for (int j = 0; j < nf; j++) s += sD[t * nf + j] * sr[b * nf + j];
