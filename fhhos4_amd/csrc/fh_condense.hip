@@ -19,8 +19,11 @@
 // and forms L^-1 [A_TF B_T] with the same broadcasts, L^-T follows, and
 // A_FF - A_TF^T X runs on v_mfma_f64_16x16x4f64 from the X left in LDS.  The
 // input is read from memory once, row by row (the bound: the nl^2 values of a
-// cell read and its blocks written).  Sums and quotients are those of the
-// column-by-column algorithm, rounding by rounding.
+// cell read and its blocks written).  The factor and the solves subtract their
+// products one by one in ascending order (the recovery's last solve in
+// descending order); A_TF^T X is summed first and then subtracted from A_FF.  A
+// cell whose quotients leave the range of div_by (an infinite diagonal entry)
+// is computed a second time with divisions.
 // Other shapes take a workgroup per cell with the matrices in LDS.
 //
 // The block pattern is formed on the device for conforming meshes (a face in
@@ -200,19 +203,15 @@ __global__ __launch_bounds__(kCondWG) void k_cell_recover(CondDev a, const doubl
 // p / nf for p < 64
 __device__ __forceinline__ int div_nf(int p, int rcp) { return (p * rcp) >> 16; }
 
-// The condensation of a cell of NC cell unknowns and m <= 63 face unknowns
-// (nfc <= 8 faces): lane r holds row r of A_TT, lane c column c of
-// [A_TF B_T] (column m: B_T).  rcp = ceil(65536 / nf); ldx: row length of X
-// in LDS, a multiple of 16 above m.
-template <int NC>
-__global__ __launch_bounds__(kCondWG, 3) void k_condense_wave(CondDev a, int rcp, int ldx) {
-    extern __shared__ double lds[];
-    const int m = a.m, nl = a.nl, nf = a.nf, nfc = a.nfc;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int cell = blockIdx.x * kCondWaves + wave;
-    if (cell >= a.ncells) return;  // wavefront-uniform; no barrier follows
-    const double* loc = a.local + (int64_t)cell * nl * nl;
-    double A[NC], x[NC];
+// x = column c of A_TT^-1 [A_TF B_T] of a cell (lane c; column m: B_T).
+// Returns whether A_TT is not positive definite or, without DIVIDE, whether a
+// quotient may have left the range of div_by: such a quotient is NaN, and a NaN
+// in a row of the factor or of x reaches x[0] or a pivot.
+template <int NC, bool DIVIDE>
+__device__ __forceinline__ bool condense_columns(const CondDev& a, const double* loc, int cell, int lane,
+                                                 double (&x)[NC]) {
+    const int m = a.m, nl = a.nl;
+    double A[NC];
     {
         const double* row = loc + (int64_t)min(lane, NC - 1) * nl;
 #pragma unroll
@@ -224,7 +223,6 @@ __global__ __launch_bounds__(kCondWG, 3) void k_condense_wave(CondDev a, int rcp
             else if (lane == m && a.BT) x[i] = a.BT[(int64_t)cell * NC + i];
         }
     }
-    const int sl = lane < nfc * nfc ? a.slot[(int64_t)cell * nfc * nfc + lane] : -1;
     // A_TT = L L^T and L^-1 [A_TF B_T] with the same broadcasts; then L^-T,
     // products in ascending order.  Lane j keeps diagonal entry j and, in rd,
     // its reciprocal.
@@ -237,8 +235,8 @@ __global__ __launch_bounds__(kCondWG, 3) void k_condense_wave(CondDev a, int rcp
             bad = true;  // wavefront-uniform
             dj = 1.0;
         }
-        const double sj = sqrt(dj), rj = 1.0 / sj, l = div_by(A[j], sj, rj);
-        x[j] = div_by(x[j], sj, rj);
+        const double sj = sqrt(dj), rj = 1.0 / sj, l = quotient<DIVIDE>(A[j], sj, rj);
+        x[j] = quotient<DIVIDE>(x[j], sj, rj);
         A[j] = lane == j ? sj : l;
         rd = lane == j ? rj : rd;
 #pragma unroll
@@ -253,17 +251,35 @@ __global__ __launch_bounds__(kCondWG, 3) void k_condense_wave(CondDev a, int rcp
             pin(x[k]);
         }
     }
-    if (bad) {
-        if (lane == 0) atomicOr(a.err, 1);
-        return;
-    }
+    if (bad) return true;
 #pragma unroll
     for (int i = NC - 1; i >= 0; i--) {
         double s = x[i];
 #pragma unroll
         for (int k = i + 1; k < NC; k++) s = fma(-bcast(A[i], k), x[k], s);
-        x[i] = div_by(s, bcast(A[i], i), bcast(rd, i));
+        x[i] = quotient<DIVIDE>(s, bcast(A[i], i), bcast(rd, i));
         pin(x[i]);
+    }
+    return !DIVIDE && __any(x[0] != x[0]);
+}
+
+// The condensation of a cell of NC cell unknowns and m <= 63 face unknowns
+// (nfc <= 8 faces): lane r holds row r of A_TT, lane c column c of
+// [A_TF B_T] (column m: B_T).  rcp = ceil(65536 / nf); ldx: row length of X
+// in LDS, a multiple of 16 above m.
+template <int NC>
+__global__ __launch_bounds__(kCondWG, 3) void k_condense_wave(CondDev a, int rcp, int ldx) {
+    extern __shared__ double lds[];
+    const int m = a.m, nl = a.nl, nf = a.nf, nfc = a.nfc;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cell = blockIdx.x * kCondWaves + wave;
+    if (cell >= a.ncells) return;  // wavefront-uniform; no barrier follows
+    const double* loc = a.local + (int64_t)cell * nl * nl;
+    const int sl = lane < nfc * nfc ? a.slot[(int64_t)cell * nfc * nfc + lane] : -1;
+    double x[NC];
+    if (condense_columns<NC, false>(a, loc, cell, lane, x) && condense_columns<NC, true>(a, loc, cell, lane, x)) {
+        if (lane == 0) atomicOr(a.err, 1);
+        return;
     }
     if (a.cstage) {
         double v = 0;
@@ -312,6 +328,32 @@ __global__ __launch_bounds__(kCondWG, 3) void k_condense_wave(CondDev a, int rcp
     }
 }
 
+// r <- A_TT^-1 r, r spread over the lanes; A: row `lane` of A_TT, P: NC^2
+// entries of the wavefront's LDS.  Returns as condense_columns does.
+template <int NC, bool DIVIDE>
+__device__ __forceinline__ bool recover_solve(double (&A)[NC], int lane, double& r, double* P) {
+    if (lane_chol<NC, false, DIVIDE>(A, 0, lane)) return true;
+    // L^-1 r with the lane's own row of L, then L^-T with its column
+    double d = 1.0;
+#pragma unroll
+    for (int j = 0; j < NC; j++)
+        if (lane == j) d = A[j];
+    const double rd = 1.0 / d;
+#pragma unroll
+    for (int j = 0; j < NC; j++) {
+        const double yj = quotient<DIVIDE>(bcast(r, j), bcast(d, j), bcast(rd, j));
+        if (lane == j) r = yj;
+        else if (lane > j) r -= A[j] * yj;
+    }
+    if (lane < NC)
+#pragma unroll
+        for (int k = 0; k < NC; k++)
+            if (k <= lane) P[lane * NC + k] = A[k];
+    lds_order();
+    r = wave_backward<NC, DIVIDE>(r, d, rd, [&](int i, int j) { return P[i * NC + j]; });
+    return !DIVIDE && __any(lane < NC && r != r);
+}
+
 // Cell unknowns of a cell of NC cell unknowns and m <= 64 face unknowns:
 // lane r holds row r of A_TT, lane p the face unknown p.
 template <int NC>
@@ -351,28 +393,19 @@ __global__ __launch_bounds__(kCondWG) void k_recover_wave(CondDev a, int rcp, co
         for (int q = 0; q < n; q++) r = fma(-ti[q], xp[q], r);
         lds_order();
     }
-    if (lane_chol<NC, false>(A, 0, lane)) {
-        if (lane == 0) atomicOr(a.err, 1);
-        return;
+    const double rhs = r;
+    if (recover_solve<NC, false>(A, lane, r, P)) {
+        // a quotient out of range: again with divisions
+        const double* row = loc + (int64_t)min(lane, NC - 1) * nl;
+#pragma unroll
+        for (int k = 0; k < NC; k++) A[k] = row[k];
+        r = rhs;
+        lds_order();
+        if (recover_solve<NC, true>(A, lane, r, P)) {
+            if (lane == 0) atomicOr(a.err, 1);
+            return;
+        }
     }
-    // L^-1 r with the lane's own row of L, then L^-T with its column
-    double d = 1.0;
-#pragma unroll
-    for (int j = 0; j < NC; j++)
-        if (lane == j) d = A[j];
-    const double rd = 1.0 / d;
-#pragma unroll
-    for (int j = 0; j < NC; j++) {
-        const double yj = div_by(bcast(r, j), bcast(d, j), bcast(rd, j));
-        if (lane == j) r = yj;
-        else if (lane > j) r -= A[j] * yj;
-    }
-    if (lane < NC)
-#pragma unroll
-        for (int k = 0; k < NC; k++)
-            if (k <= lane) P[lane * NC + k] = A[k];
-    lds_order();
-    r = wave_backward<NC>(r, d, rd, [&](int i, int j) { return P[i * NC + j]; });
     if (lane < NC) xT[(int64_t)cell * NC + lane] = r;
 }
 

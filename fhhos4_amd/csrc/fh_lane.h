@@ -48,12 +48,24 @@ __device__ __forceinline__ lane_d4 tile(lane_d4 acc, FA a, FB b) {
     return acc;
 }
 
-// a / b with r = 1 / b, correctly rounded (two residual corrections; r is
-// shared by the quotients of one divisor).
+// a / b with r = 1 / b correctly rounded, shared by the quotients of one
+// divisor: P. Markstein's method (IBM J. Res. Dev. 34, 1990).  a r is corrected
+// once to within a unit in the last place; correcting such a quotient by r
+// times its residual rounds it correctly while the residual a - b q is exact.
+// For the divisors met here (square roots, half-widths of cells: 2^-537 to
+// 2^512) that is from |a| = 2^-960 on; below, the quotient is within one unit,
+// and a zero is +0.  An infinite divisor, an infinite or NaN numerator and a
+// quotient that overflows give NaN: kernels on matrices of the caller's look for
+// NaN in their result and then start over with divisions (quotient<true>).
 __device__ __forceinline__ double div_by(double a, double b, double r) {
     double q = a * r;
     q = fma(fma(-b, q, a), r, q);
     return fma(fma(-b, q, a), r, q);
+}
+
+template <bool DIVIDE>
+__device__ __forceinline__ double quotient(double a, double b, double r) {
+    return DIVIDE ? a / b : div_by(a, b, r);
 }
 
 // Cholesky factor of an N x N matrix held as row r = lane - base in a[0..r]
@@ -62,7 +74,7 @@ __device__ __forceinline__ double div_by(double a, double b, double r) {
 // order and divided by the diagonal, as a column-by-column factorisation
 // does.  Returns whether a pivot of this lane's matrix was not positive (the
 // factorisation then goes on with 1 in its place).
-template <int N, bool GROUPS>
+template <int N, bool GROUPS, bool DIVIDE = false>
 __device__ __forceinline__ bool lane_chol(double (&a)[N], int base, int r) {
     bool bad = false;
 #pragma unroll
@@ -72,7 +84,7 @@ __device__ __forceinline__ bool lane_chol(double (&a)[N], int base, int r) {
             bad = true;
             dj = 1.0;
         }
-        const double sj = sqrt(dj), l = div_by(a[j], sj, 1.0 / sj);
+        const double sj = sqrt(dj), l = quotient<DIVIDE>(a[j], sj, 1.0 / sj);
         a[j] = r == j ? sj : l;
 #pragma unroll
         for (int k = j + 1; k < N; k++) {
@@ -125,11 +137,11 @@ __device__ __forceinline__ void lane_solve(double (&x)[N], FL l) {
 
 // x <- L^-T x for one right-hand side spread over the lanes (lane i: x_i, the
 // diagonal d of L and its reciprocal rd); l(j, i) is entry (j, i) of L.
-template <int N, class FL>
+template <int N, bool DIVIDE, class FL>
 __device__ __forceinline__ double wave_backward(double x, double d, double rd, FL l) {
     const int i = threadIdx.x & 63;
     for (int j = N - 1; j >= 0; j--) {
-        const double xj = div_by(bcast(x, j), bcast(d, j), bcast(rd, j));
+        const double xj = quotient<DIVIDE>(bcast(x, j), bcast(d, j), bcast(rd, j));
         if (i == j) x = xj;
         else if (i < j) x = fma(-l(j, i), xj, x);
     }

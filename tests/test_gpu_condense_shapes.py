@@ -116,3 +116,60 @@ def test_condense_and_recover(ctx, nc, nf, nfc, ncells, kind):
         G.condense_batched(ctx, faces, loc, nc, nf, nfaces)
     with pytest.raises(G.FhError, match="positive definite"):
         G.cell_recover_batched(ctx, faces, loc, nc, nf, nfaces, torch.from_numpy(xF).cuda())
+
+
+def _one_face_per_slot(rng, ncells, nfc, nc, nf):
+    """Cells without common faces: every block has one contribution."""
+    m = nfc * nf
+    R = rng.standard_normal((ncells, nc + m, nc + m))
+    local = 0.5 * (R + R.transpose(0, 2, 1)) + (nc + m) * np.eye(nc + m)
+    return np.arange(ncells * nfc, dtype=np.int32).reshape(ncells, nfc), local
+
+
+@pytest.mark.parametrize("nc,nf,nfc", [(1, 1, 2), (3, 2, 3), (4, 3, 6), (6, 3, 4), (10, 6, 4), (20, 10, 6), (5, 3, 5)])
+def test_infinite_diagonal_drops_the_unknown(ctx, nc, nf, nfc):
+    """A cell unknown whose diagonal entry is +Inf is eliminated with the value
+    zero: every quotient by its pivot is zero."""
+    print("case nc=%d nf=%d nfc=%d" % (nc, nf, nfc), flush=True)
+    rng = np.random.default_rng(nc)
+    ncells, m = nc, nfc * nf  # unknown c of cell c
+    faces, local = _one_face_per_slot(rng, ncells, nfc, nc, nf)
+    BT, BF, xF = rng.standard_normal((ncells, nc)), rng.standard_normal(ncells * m), rng.standard_normal(ncells * m)
+    xT, b, S = np.zeros((ncells, nc)), BF.reshape(ncells, m).copy(), []
+    for c in range(ncells):
+        local[c, c, c] = np.inf
+        keep = np.arange(nc) != c
+        TT, TF = local[c, :nc, :nc][keep][:, keep], local[c, :nc, nc:][keep]
+        S.append(local[c, nc:, nc:] - TF.T @ np.linalg.solve(TT, TF))
+        b[c] -= TF.T @ np.linalg.solve(TT, BT[c, keep])
+        xT[c, keep] = np.linalg.solve(TT, BT[c, keep] - TF @ xF[c * m:(c + 1) * m])
+    loc, bt = torch.from_numpy(local).cuda(), torch.from_numpy(BT.reshape(-1)).cuda()
+    M, bd = G.condense_batched(ctx, faces, loc, nc, nf, ncells * nfc, B_T=bt, B_F=torch.from_numpy(BF).cuda())
+    v = M.blocks()[2].reshape(ncells, nfc, nfc, nf, nf).transpose(0, 1, 3, 2, 4).reshape(ncells, m, m)
+    z = G.cell_recover_batched(ctx, faces, loc, nc, nf, ncells * nfc, torch.from_numpy(xF).cuda(), B_T=bt).cpu().numpy()
+    tol = 64 * nc * 2.3e-16
+    assert np.abs(v - np.array(S)).max() <= tol * np.abs(np.array(S)).max()
+    assert np.abs(bd.cpu().numpy().reshape(ncells, m) - b).max() <= tol * np.abs(b).max()
+    assert np.abs(z.reshape(ncells, nc) - xT).max() <= tol * max(np.abs(xT).max(), 1e-300)
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -1000, 2.0 ** 1000])
+@pytest.mark.parametrize("nc,nf,nfc", [(4, 3, 6), (20, 10, 6)])
+def test_power_of_four_scales_through(ctx, nc, nf, nfc, scale):
+    """Scaled by a power of four, every square root, quotient and product of
+    the algorithm is the unscaled one times a power of two, to the last bit."""
+    print("case nc=%d nf=%d nfc=%d scale=%g" % (nc, nf, nfc, scale), flush=True)
+    rng = np.random.default_rng(7)
+    ncells, m = 32, nfc * nf
+    faces, local = _one_face_per_slot(rng, ncells, nfc, nc, nf)
+    # no entry so small that a scaled product would be subnormal
+    local = np.where(local < 0, local - 0.5, local + 0.5)
+    BT, BF, xF = rng.standard_normal((ncells, nc)), rng.standard_normal(ncells * m), rng.standard_normal(ncells * m)
+    out = []
+    for s in (1.0, scale):
+        loc, bt, bf = (torch.from_numpy(s * a.reshape(-1)).cuda() for a in (local, BT, BF))
+        M, bd = G.condense_batched(ctx, faces, loc, nc, nf, ncells * nfc, B_T=bt, B_F=bf)
+        z = G.cell_recover_batched(ctx, faces, loc, nc, nf, ncells * nfc, torch.from_numpy(xF).cuda(), B_T=bt)
+        out.append((M.blocks()[2] / s, bd.cpu().numpy() / s, z.cpu().numpy()))
+    for a, w in zip(*out):
+        assert np.array_equal(a, w)
