@@ -176,15 +176,18 @@ double Mpnn::loss_grad(const NnGraph& g, const double* r1, const double* e1, flo
     const void* xs[2] = {diff_.p, e1};
     const void* ys[2] = {Adiff_.p, r1};
     int sl[2] = {kNnSlotE, kNnSlotE0};
-    launch_dots(c_, N, Prec::F64, 2, xs, ys, sl);
-    FH_HIP(hipMemcpyAsync(c_.h_scalars + kNnSlotE, c_.d_scalars + kNnSlotE, sizeof(double) * 2, hipMemcpyDeviceToHost,
-                          c_.stream));
+    launch_dots(c_, N, Prec::F64, 2, xs, ys, sl, true);
+    FH_HIP(hipEventRecord(scalars_.e, c_.stream));
     backward(g);
+    // the backward pass runs while the pair is looked at; grad_host stays as
+    // it is when the pair is refused
+    FH_HIP(hipEventSynchronize(scalars_.e));
+    const double E = c_.h_scalars[kNnSlotE], E0 = c_.h_scalars[kNnSlotE0];
+    if (!(E0 > 0)) c_.sync();  // nothing of a refused call is left running
+    FH_CHECK(E0 > 0, -2, "training pair with zero energy (e1^T r1 <= 0)");
     if (grad_host)
         FH_HIP(hipMemcpyAsync(grad_host, grad_.p, sizeof(float) * sh_.total(), hipMemcpyDeviceToHost, c_.stream));
     c_.sync();
-    const double E = c_.h_scalars[kNnSlotE], E0 = c_.h_scalars[kNnSlotE0];
-    FH_CHECK(E0 > 0, -2, "training pair with zero energy (e1^T r1 <= 0)");
     return E / E0;
 }
 

@@ -81,6 +81,13 @@ private:
     int step_ = 0;
     int cap_ = 0;
     DevBuf v_, u_, x0_, gy_, h_, m_, dh_, diff_, Adiff_;
+    struct Event {
+        hipEvent_t e = nullptr;
+        Event() { FH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming)); }
+        ~Event() { (void)hipEventDestroy(e); }
+        Event(const Event&) = delete;
+        Event& operator=(const Event&) = delete;
+    } scalars_;  // loss_grad: the loss has reached the host
     // delta into out, or e1 - delta when e1 is not null
     void forward(const NnGraph& g, const double* r1, const double* e1, double* out, bool bf16);
     void backward(const NnGraph& g);

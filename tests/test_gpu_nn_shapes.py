@@ -45,3 +45,29 @@ def test_network_matches_oracle(mesh, n, k, layers):
     loss, grad = nn.loss_grad(g, torch.from_numpy(r1).cuda(), torch.from_numpy(e1).cuda())
     assert abs(loss - loss_ref) <= 1e-4 * abs(loss_ref)
     assert np.abs(grad - grad_ref).max() <= 2e-4 * np.abs(grad_ref).max()
+
+
+def test_refused_pair_leaves_the_gradient_buffer():
+    """A pair without energy is refused before anything is written to the
+    caller's gradient, and the network works on as before."""
+    import ctypes as C
+
+    ctx = G.Context(0)
+    P = G.HhoProblem(dim=2, mesh="quad", n=6, k=1, perturb=0.15, seed=3)
+    g = G.NnGraph(ctx, P.matrix(ctx, keep_host=True), G.face_features(P))
+    nn = G.Mpnn(ctx, P.nf, layers=2, seed=11)
+    rng = np.random.default_rng(6)
+    e1 = rng.standard_normal(P.n_unknowns)
+    pair = [torch.from_numpy(v).cuda() for v in (P.scipy() @ e1, e1)]
+    loss, grad = nn.loss_grad(g, *pair)
+    zero = torch.zeros_like(pair[0])
+    torch.cuda.synchronize()
+    buf = np.full(nn.num_params(), 7.0, dtype=np.float32)
+    value = C.c_double(7.0)
+    for r, e in [(zero, zero), (zero, pair[1]), (-pair[0], pair[1])]:
+        torch.cuda.synchronize()
+        rc = G.lib().fh_nn_loss_grad(ctx.h, nn.h, g.h, r.data_ptr(), e.data_ptr(), C.byref(value), buf.ctypes.data)
+        assert rc == -2 and value.value == 7.0
+        assert np.all(buf == 7.0)
+    loss2, grad2 = nn.loss_grad(g, *pair)
+    assert loss2 == loss and np.array_equal(grad, grad2)
