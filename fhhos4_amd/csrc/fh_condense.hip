@@ -111,9 +111,37 @@ __device__ void chol_solve_col(const double* L, int nc, double* Y, int ld, int c
     }
 }
 
+// Schur entries A_FF - A_TF^T X of a workgroup's cell on the matrix cores: 16 x
+// 16 output tiles dealt to the wavefronts, four cell unknowns per instruction
+// (zero beyond nc and m).  T: A_TF (nc x m), X: nc x (m + 1), in LDS.
+__device__ void schur_tiles(const CondDev& a, const double* T, const double* X, const double* loc, const int* slot) {
+    const int nc = a.nc, m = a.m, nl = a.nl, nf = a.nf, nfc = a.nfc;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane >> 4, lc = lane & 15, tiles = (m + 15) / 16;
+    for (int t = wave; t < tiles * tiles; t += kCondWaves) {
+        const int ti = t / tiles, tj = t - ti * tiles, pa = 16 * ti + lc, q = 16 * tj + lc;
+        lane_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        for (int k0 = 0; k0 < nc; k0 += 4) {
+            const int k = k0 + lr;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k < nc && pa < m ? T[k * m + pa] : 0.0,
+                                                       k < nc && q < m ? X[k * (m + 1) + q] : 0.0, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int p = 16 * ti + lr + 4 * v;
+            if (p >= m || q >= m) continue;
+            const int s = slot[(p / nf) * nfc + q / nf];
+            if (s == -1) continue;
+            add_entry(a.vals, s, nf * nf, (p % nf) * nf + q % nf, loc[(int64_t)(nc + p) * nl + nc + q] - acc[v]);
+        }
+    }
+}
+
 // Other shapes: a workgroup per cell, the matrices in LDS (nc^2 + nc m +
 // nc (m + 1) doubles), the factorisation column by column with barriers, the
-// triangular solves a column per thread, the Schur blocks entry by entry.
+// triangular solves a column per thread, the Schur blocks by tiles (MFMA) or
+// entry by entry.
+template <bool MFMA>
 __global__ __launch_bounds__(kCondWG) void k_condense(CondDev a) {
     extern __shared__ double lds[];
     const int nc = a.nc, m = a.m, nl = a.nl, nf = a.nf, nfc = a.nfc;
@@ -138,13 +166,17 @@ __global__ __launch_bounds__(kCondWG) void k_condense(CondDev a) {
     __syncthreads();
     // Schur entries (p, q) of the cell's faces j1 = p / nf, j2 = q / nf
     const int* slot = a.slot + (int64_t)cell * nfc * nfc;
-    for (int t = threadIdx.x; t < m * m; t += blockDim.x) {
-        const int p = t / m, q = t - p * m;
-        const int s = slot[(p / nf) * nfc + q / nf];
-        if (s == -1) continue;
-        double v = loc[(int64_t)(nc + p) * nl + nc + q];
-        for (int r = 0; r < nc; r++) v -= T[r * m + p] * X[r * (m + 1) + q];
-        add_entry(a.vals, s, nf * nf, (p % nf) * nf + q % nf, v);
+    if constexpr (MFMA) {
+        schur_tiles(a, T, X, loc, slot);
+    } else {
+        for (int t = threadIdx.x; t < m * m; t += blockDim.x) {
+            const int p = t / m, q = t - p * m;
+            const int s = slot[(p / nf) * nfc + q / nf];
+            if (s == -1) continue;
+            double v = loc[(int64_t)(nc + p) * nl + nc + q];
+            for (int r = 0; r < nc; r++) v -= T[r * m + p] * X[r * (m + 1) + q];
+            add_entry(a.vals, s, nf * nf, (p % nf) * nf + q % nf, v);
+        }
     }
     if (a.cstage) {
         for (int p = threadIdx.x; p < m; p += blockDim.x) {
@@ -600,9 +632,13 @@ static void launch_condense(Ctx& c, const CondDev& d) {
                                dim3(kCondWG), lds, c.stream, d, (65536 + d.nf - 1) / d.nf, ldx);
         });
     } else {
+        // on the matrix cores where the blocks fill 2 x 2 tiles and two steps of
+        // four cell unknowns: 4096 cells of nc = 35, m = 90 take 1193 us (1347 us
+        // entry by entry), of nc = 20, m = 80 348 us (414 us)
         const size_t lds = cond_lds_bytes(d.nc, d.m);
-        set_lds((const void*)k_condense, lds);
-        hipLaunchKernelGGL(k_condense, dim3(d.ncells), dim3(kCondWG), lds, c.stream, d);
+        auto kern = d.m >= 32 && d.nc >= 8 && mfma_enabled() ? k_condense<true> : k_condense<false>;
+        set_lds((const void*)kern, lds);
+        hipLaunchKernelGGL(kern, dim3(d.ncells), dim3(kCondWG), lds, c.stream, d);
     }
     FH_HIP(hipGetLastError());
 }

@@ -9,6 +9,8 @@ built on the host, and sums of several contributions).
 Tolerance: a block entry is a sum of nc products per contribution after a
 backward-stable solve with condition number below 2: 64 nc units in the last
 place of the largest entry bound it amply."""
+from fractions import Fraction
+
 import numpy as np
 import pytest
 
@@ -56,7 +58,7 @@ def _faces(rng, ncells, nfc, kind):
 CASES = [(nc, nf, nfc, n, "plain") for nc, nf, nfc, n in
          [(1, 1, 1, 1), (1, 1, 6, 5), (3, 2, 3, 9), (4, 3, 6, 6), (6, 3, 4, 7), (10, 6, 4, 3), (10, 4, 4, 10),
           (20, 10, 6, 4), (20, 10, 4, 5), (20, 9, 7, 3), (3, 2, 8, 11), (1, 16, 1, 3),
-          (2, 2, 4, 3), (5, 3, 5, 3), (20, 10, 7, 2), (4, 3, 9, 3)]] + \
+          (2, 2, 4, 3), (5, 3, 5, 3), (20, 10, 7, 2), (4, 3, 9, 3), (35, 15, 6, 3), (8, 4, 8, 5), (9, 3, 11, 3)]] + \
         [(4, 3, 6, 6, "three"), (10, 6, 4, 5, "twice"), (2, 3, 4, 5, "three"), (20, 10, 6, 3, "twice")]
 
 
@@ -173,3 +175,30 @@ def test_power_of_four_scales_through(ctx, nc, nf, nfc, scale):
         out.append((M.blocks()[2] / s, bd.cpu().numpy() / s, z.cpu().numpy()))
     for a, w in zip(*out):
         assert np.array_equal(a, w)
+
+
+@pytest.mark.parametrize("nc,nf,nfc", [(8, 4, 8), (9, 4, 8), (20, 8, 8), (35, 15, 6)])
+def test_large_shapes_run_on_the_matrix_cores(ctx, nc, nf, nfc):
+    """Shapes beyond one wavefront's with 32 face unknowns or more: with A_TT = I
+    the solves are exact and a block entry is A_FF minus the product A_TF^T A_TF
+    that the matrix instruction forms, a chain of fused multiply-adds over
+    ascending cell unknowns.  Entry by entry the products are subtracted from
+    A_FF one after the other, which rounds differently."""
+    rng = np.random.default_rng(nc)
+    m = nf * nfc
+    local = rng.standard_normal((1, nc + m, nc + m))
+    local[0, :nc, :nc] = np.eye(nc)
+    T, FF = local[0, :nc, nc:], local[0, nc:, nc:]
+    faces = np.arange(nfc, dtype=np.int32).reshape(1, nfc)
+    M, _ = G.condense_batched(ctx, faces, torch.from_numpy(local).cuda(), nc, nf, nfc)
+    v = M.blocks()[2].reshape(nfc, nfc, nf, nf).transpose(0, 2, 1, 3).reshape(m, m)
+    same = 0
+    for p, q in rng.integers(0, m, (200, 2)):
+        acc, one = 0.0, float(FF[p, q])
+        for k in range(nc):
+            t = Fraction(T[k, p]) * Fraction(T[k, q])
+            acc = float(t + Fraction(acc))
+            one = float(Fraction(one) - t)
+        assert v[p, q] == FF[p, q] - acc
+        same += one == FF[p, q] - acc
+    assert same < 200  # the two orders can be told apart
