@@ -651,58 +651,59 @@ struct HostPattern {
     std::vector<unsigned char> multi;
 };
 
+// Face by face from the (cell, local face) entries of every face: one sorted
+// list at a time, in place of a list per face (4096 cells of 12 faces: 6.9 ms a
+// call with those and a separate search for every block).
 void host_pattern(int ncells, int nfc, int nfaces, const int* cell_faces, Bcsr& A, HostPattern& H) {
-    // every pair of system faces of one cell, sorted columns
-    std::vector<std::vector<int>> adj(nfaces);
-    for (int e = 0; e < ncells; e++)
-        for (int j1 = 0; j1 < nfc; j1++) {
-            const int f1 = cell_faces[(int64_t)e * nfc + j1];
-            if (f1 < 0) continue;
-            for (int j2 = 0; j2 < nfc; j2++) {
-                const int f2 = cell_faces[(int64_t)e * nfc + j2];
-                if (f2 >= 0) adj[f1].push_back(f2);
+    const int64_t nent = (int64_t)ncells * nfc;
+    // entries of every face, in cell order
+    std::vector<int64_t> ptr((size_t)nfaces + 1, 0);
+    for (int64_t t = 0; t < nent; t++)
+        if (cell_faces[t] >= 0) ptr[cell_faces[t] + 1]++;
+    for (int f = 0; f < nfaces; f++) ptr[f + 1] += ptr[f];
+    std::vector<int64_t> ent(ptr[nfaces]), fill(ptr.begin(), ptr.end() - 1);
+    for (int64_t t = 0; t < nent; t++)
+        if (cell_faces[t] >= 0) ent[fill[cell_faces[t]]++] = t;
+    A.h_rowptr.assign((size_t)nfaces + 1, 0);
+    A.h_colidx.clear();
+    H.multi.clear();
+    H.slot.assign((size_t)nent * nfc, -1);
+    std::vector<int> row;
+    for (int f = 0; f < nfaces; f++) {
+        // the distinct faces of the cells of f, ascending
+        row.clear();
+        for (int64_t e = ptr[f]; e < ptr[f + 1]; e++)
+            for (int j = 0; j < nfc; j++) {
+                const int g = cell_faces[ent[e] / nfc * nfc + j];
+                if (g >= 0) row.push_back(g);
+            }
+        std::sort(row.begin(), row.end());
+        const size_t base = A.h_colidx.size();
+        for (size_t i = 0; i < row.size(); i++) {
+            if (i > 0 && row[i] == row[i - 1]) {
+                H.multi.back() = 1;
+            } else {
+                A.h_colidx.push_back(row[i]);
+                H.multi.push_back(0);
             }
         }
-    A.h_rowptr.assign(nfaces + 1, 0);
-    std::vector<unsigned char>& multi = H.multi;
-    for (int f = 0; f < nfaces; f++) {
-        auto& v = adj[f];
-        std::sort(v.begin(), v.end());
-        for (size_t i = 0; i < v.size(); i++) {
-            if (i > 0 && v[i] == v[i - 1]) multi.back() = 1;
-            else multi.push_back(0);
-        }
-        v.erase(std::unique(v.begin(), v.end()), v.end());
-        FH_CHECK((int64_t)A.h_rowptr[f] + (int64_t)v.size() < INT32_MAX, -2, "too many blocks");
-        A.h_rowptr[f + 1] = A.h_rowptr[f] + (int)v.size();
+        FH_CHECK(A.h_colidx.size() < (size_t)INT32_MAX, -2, "too many blocks");
+        A.h_rowptr[f + 1] = (int)A.h_colidx.size();
+        // block of every face pair (f, g) of the cells
+        const auto b0 = A.h_colidx.begin() + base;
+        for (int64_t e = ptr[f]; e < ptr[f + 1]; e++)
+            for (int j = 0; j < nfc; j++) {
+                const int g = cell_faces[ent[e] / nfc * nfc + j];
+                if (g < 0) continue;
+                const int p = (int)(std::lower_bound(b0, A.h_colidx.end(), g) - A.h_colidx.begin());
+                H.slot[(size_t)ent[e] * nfc + j] = H.multi[p] ? -2 - p : p;
+            }
     }
     A.nnzb = A.h_rowptr[nfaces];
     A.h_colidx.resize(std::max<int64_t>(1, A.nnzb));
-    for (int f = 0; f < nfaces; f++) std::copy(adj[f].begin(), adj[f].end(), A.h_colidx.begin() + A.h_rowptr[f]);
-    // block index of every (cell, j1, j2)
-    H.slot.assign((size_t)ncells * nfc * nfc, -1);
-    for (int e = 0; e < ncells; e++)
-        for (int j1 = 0; j1 < nfc; j1++) {
-            const int f1 = cell_faces[(int64_t)e * nfc + j1];
-            if (f1 < 0) continue;
-            const int* b0 = A.h_colidx.data() + A.h_rowptr[f1];
-            const int* b1 = A.h_colidx.data() + A.h_rowptr[f1 + 1];
-            for (int j2 = 0; j2 < nfc; j2++) {
-                const int f2 = cell_faces[(int64_t)e * nfc + j2];
-                if (f2 < 0) continue;
-                const int p = (int)(std::lower_bound(b0, b1, f2) - A.h_colidx.data());
-                H.slot[((size_t)e * nfc + j1) * nfc + j2] = multi[p] ? -2 - p : p;
-            }
-        }
-    // (cell, local face) entries of every face, in cell order
-    H.fptr.assign(nfaces + 1, 0);
-    for (int64_t t = 0; t < (int64_t)ncells * nfc; t++)
-        if (cell_faces[t] >= 0) H.fptr[cell_faces[t] + 1]++;
-    for (int f = 0; f < nfaces; f++) H.fptr[f + 1] += H.fptr[f];
-    H.fent.resize(std::max(1, H.fptr[nfaces]));
-    std::vector<int> fill(H.fptr.begin(), H.fptr.end() - 1);
-    for (int64_t t = 0; t < (int64_t)ncells * nfc; t++)
-        if (cell_faces[t] >= 0) H.fent[fill[cell_faces[t]]++] = (int)t;
+    H.fptr.assign(ptr.begin(), ptr.end());
+    H.fent.assign(ent.begin(), ent.end());
+    H.fent.resize(std::max<size_t>(1, H.fent.size()));
 }
 
 }  // namespace
