@@ -92,6 +92,9 @@ int fh_ctx_destroy(fh_ctx* ctx) {
 int fh_ctx_sync(fh_ctx* ctx) {
     return guard([&] { NEED(ctx); ctx->c.sync(); });
 }
+int fh_release_memory(void) {
+    return guard([&] { fh::kept_trim(); });
+}
 
 int fh_mat_from_csr(fh_ctx* ctx, int nrows, int ncols, int bs, const int* rowptr, const int* colidx,
                     const double* vals, int keep_host, fh_mat** out) {

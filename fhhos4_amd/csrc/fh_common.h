@@ -66,12 +66,16 @@ struct Ctx {
 // 0.26 ms in hipFree, and a program that allocates and frees one in every
 // call has, after some hundred calls, gone once through the card's memory:
 // from then on each call waits 8 to 30 ms for the driver to clear what was
-// freed.  At most kKeptBytes stay; they are freed oldest first, when an
-// allocation fails, and with the last context of the process.
-constexpr size_t kKeptMin = (size_t)1 << 20, kKeptBytes = (size_t)4 << 30;
+// freed.  At most kKeptShare of the device's memory stays (the oldest are
+// freed first); all are freed when an allocation of the library fails, by
+// fh_release_memory() and with the last context of the process.  Up to 1 MiB
+// hipMalloc and hipFree take 0.7 us each, from 4 MiB on 12 us.
+constexpr size_t kKeptMin = (size_t)1 << 20, kKeptShare = 128;
 void* kept_take(size_t bytes, int dev, size_t* cap);  // null: none fits
 void kept_give(void* p, size_t cap, int dev);
 void kept_trim();
+// hipMalloc; frees the kept buffers and tries again when memory has run out.
+void* device_malloc(size_t bytes);
 
 // Owning device allocation.
 struct DevBuf {
@@ -125,17 +129,9 @@ struct DevBuf {
 
 private:
     void allocate(size_t b) {
-        hipError_t e = hipMalloc(&p, b);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            kept_trim();
-            e = hipMalloc(&p, b);
-        }
-        if (e != hipSuccess) {
-            p = nullptr;
-            bytes = 0;
-        }
-        FH_HIP(e);
+        bytes = 0;  // nothing is held if this throws
+        p = device_malloc(b);
+        bytes = b;
     }
 };
 

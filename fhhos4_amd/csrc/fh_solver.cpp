@@ -26,12 +26,15 @@ struct Kept {
     void* p;
     size_t cap;
     int dev;
+    uint64_t given;  // number of the release
 };
 struct KeptList {
     std::mutex lock;
     std::vector<Kept> free;  // oldest first
-    size_t total = 0;
+    size_t total = 0, limit = 0;
     int contexts = 0;
+    uint64_t gives = 0;
+    std::vector<uint64_t> idle;  // per device: no work uses what was released up to here
 };
 // never destroyed: buffers may be released during the process's exit
 KeptList& kept_list() {
@@ -43,6 +46,7 @@ KeptList& kept_list() {
 void* kept_take(size_t bytes, int dev, size_t* cap) {
     KeptList& l = kept_list();
     Kept k{};
+    uint64_t upto;
     {
         std::lock_guard<std::mutex> g(l.lock);
         size_t best = l.free.size();
@@ -55,14 +59,23 @@ void* kept_take(size_t bytes, int dev, size_t* cap) {
         k = l.free[best];
         l.free.erase(l.free.begin() + best);
         l.total -= k.cap;
+        if ((size_t)dev < l.idle.size() && k.given <= l.idle[dev]) {
+            *cap = k.cap;
+            return k.p;
+        }
+        upto = l.gives;
     }
     // work of any stream that still uses the buffer ends first (hipFree waits
-    // in the same way)
+    // in the same way); it was issued before the release, so what has been
+    // released up to here is idle then too
     if (hipDeviceSynchronize() != hipSuccess) {
         (void)hipGetLastError();
         kept_give(k.p, k.cap, dev);
         return nullptr;
     }
+    std::lock_guard<std::mutex> g(l.lock);
+    if (l.idle.size() <= (size_t)dev) l.idle.resize(dev + 1, 0);
+    l.idle[dev] = std::max(l.idle[dev], upto);
     *cap = k.cap;
     return k.p;
 }
@@ -72,13 +85,14 @@ void kept_give(void* p, size_t cap, int dev) {
     std::vector<Kept> out;
     {
         std::lock_guard<std::mutex> g(l.lock);
-        if (cap > kKeptBytes || l.contexts == 0) {
-            out.push_back({p, cap, dev});
+        const Kept k{p, cap, dev, ++l.gives};
+        if (cap > l.limit || l.contexts == 0) {
+            out.push_back(k);
         } else {
-            l.free.push_back({p, cap, dev});
+            l.free.push_back(k);
             l.total += cap;
             size_t n = 0;
-            while (l.total > kKeptBytes) l.total -= l.free[n++].cap;
+            while (l.total > l.limit) l.total -= l.free[n++].cap;
             out.assign(l.free.begin(), l.free.begin() + n);
             l.free.erase(l.free.begin(), l.free.begin() + n);
         }
@@ -97,13 +111,27 @@ void kept_trim() {
     for (const Kept& k : out) (void)hipFree(k.p);
 }
 
-static void count_context(int change) {
+void* device_malloc(size_t bytes) {
+    void* p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        kept_trim();
+        e = hipMalloc(&p, bytes);
+    }
+    FH_HIP(e);
+    return p;
+}
+
+// A context on a device with `memory` bytes comes, or one goes (0).
+static void count_context(int change, size_t memory) {
     KeptList& l = kept_list();
     bool last;
     {
         std::lock_guard<std::mutex> g(l.lock);
         l.contexts += change;
         last = l.contexts == 0;
+        if (memory) l.limit = l.limit ? std::min(l.limit, memory / kKeptShare) : memory / kKeptShare;
     }
     if (last) kept_trim();
 }
@@ -115,13 +143,15 @@ Ctx::Ctx(int dev) : device(dev) {
     }
     FH_HIP(hipSetDevice(dev));
     FH_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    FH_HIP(hipMalloc(&d_partials, sizeof(double) * kMaxPartials * kPartialSlots));
-    FH_HIP(hipMalloc(&d_scalars, sizeof(double) * kScalars));
+    d_partials = (double*)device_malloc(sizeof(double) * kMaxPartials * kPartialSlots);
+    d_scalars = (double*)device_malloc(sizeof(double) * kScalars);
     FH_HIP(hipHostMalloc(&h_scalars, sizeof(double) * kScalars, hipHostMallocDefault));
     FH_HIP(hipMemsetAsync(d_scalars, 0, sizeof(double) * kScalars, stream));
     FH_HIP(hipStreamSynchronize(stream));
     noalloc_scratch_init(dev);  // this device is current
-    count_context(1);
+    size_t free_bytes = 0, memory = 0;
+    FH_HIP(hipMemGetInfo(&free_bytes, &memory));
+    count_context(1, memory);
 }
 
 Ctx::~Ctx() {
@@ -131,7 +161,7 @@ Ctx::~Ctx() {
     if (d_scalars) (void)hipFree(d_scalars);
     if (h_scalars) (void)hipHostFree(h_scalars);
     if (stream) (void)hipStreamDestroy(stream);
-    count_context(-1);
+    count_context(-1, 0);
 }
 
 static void dot1(Ctx& c, int64_t n, Prec p, const void* x, const void* y, int slot, bool to_host = false) {

@@ -53,6 +53,7 @@ _SIGS = {
     "fh_ctx_create": [C.c_int, _pp],
     "fh_ctx_destroy": [_vp],
     "fh_ctx_sync": [_vp],
+    "fh_release_memory": [],
     "fh_mat_from_csr": [_vp, C.c_int, C.c_int, C.c_int, _i32p, _i32p, _f64p, C.c_int, _pp],
     "fh_mat_from_blocks": [_vp, C.c_int, C.c_int, C.c_int, _i32p, _i32p, _f64p, C.c_int, _pp],
     "fh_mat_convert": [_vp, _vp, C.c_int, _pp],
@@ -419,6 +420,12 @@ def residual(ctx, A, b, x, r):
     pb = _dev(b, n, like=x, name="b")
     pr = _dev(r, n, like=x, name="r")
     _check(lib().fh_residual(ctx.h, A.h, pb, px, pr, _vprec(x)))
+
+
+def release_memory():
+    """Frees the device memory that the library keeps for its next assembly or
+    condensation (fh_release_memory), for other allocators of the process."""
+    _check(lib().fh_release_memory())
 
 
 @_ordered

@@ -32,6 +32,14 @@ enum { FH_F64 = 0, FH_F32 = 1, FH_BF16 = 2 };
 int fh_ctx_create(int device, fh_ctx** out);
 int fh_ctx_destroy(fh_ctx* ctx);
 int fh_ctx_sync(fh_ctx* ctx);
+/* Frees the device memory that the library keeps for its next calls.  Buffers
+ * of 1 MiB and more of the operators made by fh_hho_assemble_gpu and
+ * fh_condense_batched (block columns and values, element layout) and of those
+ * calls' own work stay allocated when they are released, for the next such
+ * call: at most 1/128 of the device's memory, and none after the last context
+ * is destroyed.  An allocation of the library that fails frees them by itself;
+ * call this before another allocator of the process needs the memory. */
+int fh_release_memory(void);
 /* Error reporting; replaces Utils::FatalError (src/Utils/Utils.h:258-263). */
 const char* fh_last_error(void);
 

@@ -50,3 +50,27 @@ def test_condensation_again():
             # a block of two cells is the sum of two terms in either order
             assert np.array_equal(want[k], v)
         want[k] = v
+
+
+def _used():
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    return total - free, total
+
+
+def test_kept_memory_is_bounded_and_released():
+    ctx = G.Context(0)
+    P = G.HhoProblem(dim=3, mesh="hex", n=20, k=3, perturb=0.15, seed=1, defer_assembly=True)
+    P.assemble_gpu(ctx)  # what the first call sets up for good
+    G.release_memory()
+    used, total = _used()
+    held = [P.assemble_gpu(ctx)[0] for _ in range(12)]  # 0.3 GB each
+    assert _used()[0] - used > total // 128 + (1 << 29)
+    del held
+    torch.cuda.empty_cache()
+    kept = _used()[0] - used
+    slack = 64 << 20
+    assert kept <= total // 128 + slack
+    G.release_memory()
+    assert _used()[0] - used <= slack
+    G.release_memory()  # nothing left to free
