@@ -1021,6 +1021,7 @@ void Solver::Solve(const double* b, double* x, bool x_is_zero) {
     auto t0 = std::chrono::steady_clock::now();
     hist_.clear();
     if (nn_) {
+        FH_CHECK(nn_counters_.p != nullptr, -2, "the learned post-smoother must be set before Setup()");
         launch_fill(c_, 2, nn_counters_.p, Prec::F32, 0.0);  // two int zeros (same bit pattern as 0.0f)
         nn_fallbacks_seen_ = 0;
     }
@@ -1087,13 +1088,10 @@ void Solver::solve_cg(const double* b, double* x, bool xz) {
     hist_.push_back(res);
     stats_.converged = 0;
     auto stop = FH_STOP_TEST();
-    auto precondition = [&] {
-        apply_prec(r_, z_, nullptr);
-        dot1(c_, n, P, r_.data(), z_.data(), rz[it % 2]);
-    };
     while (!stop()) {
         if (it > 0) {
-            if (!nn_) precondition();
+            apply_prec(r_, z_, nullptr);
+            dot1(c_, n, P, r_.data(), z_.data(), rz[it % 2]);
             launch_axpby(c_, n, P, z_.data(), d_.data(), 1.0, -1, -1, 1.0, rz[it % 2], rz[(it + 1) % 2]);  // d = z + beta d
         }
         launch_bcsr(c_, *A_, OP_SPMV, P, d_.data(), nullptr, Ad_.data(), 1.0, 0.0, 0.0, nullptr, P, nullptr, 0);
@@ -1101,9 +1099,7 @@ void Solver::solve_cg(const double* b, double* x, bool xz) {
         launch_cg_update_rr(c_, n, (double*)x, (const double*)d_.data(), (double*)r_.data(), (const double*)Ad_.data(),
                             rz[it % 2], S_DAD, 1.0, S_RR, true);
         it++;
-        // |r| decides before the next preconditioner application, except that
-        // the learned post-smoother counts one after the last iteration too
-        if (nn_) precondition();
+        // |r| decides before the next preconditioner application
         double rr = read_scalar(S_RR);
         res = bn > 0 ? std::sqrt(rr) / bn : std::sqrt(rr);
         hist_.push_back(res);

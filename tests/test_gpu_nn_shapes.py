@@ -71,3 +71,17 @@ def test_refused_pair_leaves_the_gradient_buffer():
         assert np.all(buf == 7.0)
     loss2, grad2 = nn.loss_grad(g, *pair)
     assert loss2 == loss and np.array_equal(grad, grad2)
+
+
+@pytest.mark.parametrize("solver", ["fcg", "cg"])
+def test_network_set_after_setup_is_refused(solver):
+    """Setup allocates what the learned post-smoother works on."""
+    ctx = G.Context(0)
+    P = G.HhoProblem(dim=2, mesh="quad", n=6, k=1, perturb=0.15, seed=3)
+    A = P.matrix(ctx, keep_host=True)
+    s = G.Solver(ctx, solver=solver, prec="bj")
+    s.setup(A)
+    s.set_learned_smoother(G.Mpnn(ctx, P.nf, layers=2, seed=11), G.NnGraph(ctx, A, G.face_features(P)))
+    b = torch.from_numpy(P.rhs()).cuda()
+    with pytest.raises(G.FhError, match="before Setup"):
+        s.solve(b, torch.zeros_like(b))
