@@ -70,7 +70,7 @@ struct Ctx {
 // freed first); all are freed when an allocation of the library fails, by
 // fh_release_memory() and with the last context of the process.  Up to 1 MiB
 // hipMalloc and hipFree take 0.7 us each, from 4 MiB on 12 us.
-constexpr size_t kKeptMin = (size_t)1 << 20, kKeptShare = 128;
+constexpr size_t kKeptMin = (size_t)1 << 20, kKeptShare = 72;
 void* kept_take(size_t bytes, int dev, size_t* cap);  // null: none fits
 void kept_give(void* p, size_t cap, int dev);
 void kept_trim();

@@ -36,7 +36,7 @@ int fh_ctx_sync(fh_ctx* ctx);
  * of 1 MiB and more of the operators made by fh_hho_assemble_gpu and
  * fh_condense_batched (block columns and values, element layout) and of those
  * calls' own work stay allocated when they are released, for the next such
- * call: at most 1/128 of the device's memory, and none after the last context
+ * call: at most 1/72 of the device's memory, and none after the last context
  * is destroyed.  An allocation of the library that fails frees them by itself;
  * call this before another allocator of the process needs the memory. */
 int fh_release_memory(void);

@@ -64,13 +64,13 @@ def test_kept_memory_is_bounded_and_released():
     P.assemble_gpu(ctx)  # what the first call sets up for good
     G.release_memory()
     used, total = _used()
-    held = [P.assemble_gpu(ctx)[0] for _ in range(12)]  # 0.3 GB each
-    assert _used()[0] - used > total // 128 + (1 << 29)
+    held = [P.assemble_gpu(ctx)[0] for _ in range(20)]  # 0.3 GB each
+    assert _used()[0] - used > total // 72 + (1 << 29)
     del held
     torch.cuda.empty_cache()
     kept = _used()[0] - used
     slack = 64 << 20
-    assert kept <= total // 128 + slack
+    assert kept <= total // 72 + slack
     G.release_memory()
     assert _used()[0] - used <= slack
     G.release_memory()  # nothing left to free
