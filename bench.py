@@ -245,8 +245,8 @@ def condense_bench(args, G, np, torch):
     byt = ncells * (nl * nl * 8 + nc * 8 + nfc * nfc * nf * nf * 8 * 2)
     out = {"kernel": "condense_batched", "cells": ncells, "faces": nfaces, "nc": nc, "face_unknowns": nfc * nf,
            "call_s": float(np.median(ts)), "flop": flop, "bytes": byt,
-           "note": "call time includes the host block pattern; the kernel's own duration is in the rocprof summary"}
-    log("condensation of %d cells (%d faces): %.3f s per call (pattern on the host, kernel, right-hand side)"
+           "note": "call time includes the block pattern and the copies; the kernel's own duration is in the rocprof summary"}
+    log("condensation of %d cells (%d faces): %.3f s per call (pattern, kernel, right-hand side)"
         % (ncells, nfaces, out["call_s"]))
     print(json.dumps(out), flush=True)
 

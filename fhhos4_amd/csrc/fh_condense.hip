@@ -37,9 +37,10 @@
 //
 // MI355X, hexahedra at k = 3 (nc = 20, 60 face unknowns), 13 824 cells, the
 // condensation and the recovery of all cells: 0.74 ms, of which the cells'
-// condensation 286 us (3.2 TB/s of the values read and the blocks written; its
-// registers leave three wavefronts per SIMD to cover the loads) and the
-// recovery 80 us.  A workgroup per cell with a barrier per column and the
+// condensation 287 us and the recovery 80 us.  Bound by memory: 110 592 cells
+// take 2.34 ms for 7.4 GB (3.2 TB/s), and the counters show 11.3 GB (4.9 TB/s):
+// A_TF is read three times and does not stay in the caches; its registers
+// leave three wavefronts per SIMD to cover the loads.  A workgroup per cell with a barrier per column and the
 // pattern formed on the host by sorting took 6.2 ms.
 #include <algorithm>
 #include <cstdlib>
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(kCondWG, 3) void k_condense_wave(CondDev a, int rcp
 #pragma unroll
         for (int i = 0; i < NC; i++) X[i * ldx + lane] = x[i];
     lds_order();
-    // A_FF - A_TF^T X by 16 x 16 tiles, A_TF read again (from L2); columns of
+    // A_FF - A_TF^T X by 16 x 16 tiles, A_TF read again; columns of
     // eliminated faces and beyond m reach entries that are not stored only
     const int lr = lane >> 4, lc = lane & 15, T = (m + 15) >> 4;
     constexpr int ST = (NC + 3) / 4;

@@ -12,7 +12,9 @@ struct HhoDev {
     const int* cv;                 // cell vertices (nvc per cell)
     const int* cf;                 // cell faces (nfc per cell)
     const int* fv;                 // face vertices (nvf per face)
-    const double* K;               // diffusion tensor, 9 per cell
+    // diffusion tensor, 9 per cell; general cells (kind 2) take diagonal ones
+    // only, as every kappa field of fh_hho.cpp is, and refuse others
+    const double* K;
     const int* cft;                // face table of every (cell, local face)
     const double* Shat;            // 9 x nr x nr reference stiffness tensors
     const double* cellPsi;         // nq x nr reconstruction basis at the cell rule

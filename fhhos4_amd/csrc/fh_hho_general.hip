@@ -26,9 +26,9 @@
 //
 // MI355X, hexahedra at k = 3: 13 824 cells in 4.84 ms (0.35 us per cell; the
 // products alone would take 0.1 us at the rate of a large FP64 matrix
-// product).  Bound by latency: of 330 000 cycles per cell, with two cells in
-// flight per CU, 35% go to the gradient products, 16% to the face integrals,
-// 15% to the factorisation of S and the solves with it.  A workgroup of 256
+// product).  Bound by latency: of 397 000 cycles per cell, with two cells in
+// flight per CU, 33% go to the gradient products, 14% to the face integrals,
+// 12% to the factorisation of S and the solves with it.  A workgroup of 256
 // threads per cell with an entry per thread and a barrier per column took
 // 48 ms (146 KB of LDS: one cell per CU).  k = 2: 1.11 ms for 12 167 cells.
 #include "fh_hho_eval.h"

@@ -1985,9 +1985,15 @@ bool launch_cheb_start(Ctx& c, const Bcsr& A, Prec vprec, const void* x, const v
     if (A.sliced_state == 0 && !c.no_alloc) sliced_decide(c, A);
     // The correction on SELL-64 levels stays a pass of its own: 26 167 rows
     // (FP64) take 8.4 us fused and 5.3 + 3.2 us apart, 95 232 rows 10.0 us and
-    // 6.2 + 3.1 us; 7 663 rows in CSR take 4.6 us and 3.4 + 3.0 us.  The start
-    // from zero takes 7.8 us for 6.2 + 4.6 us at 95 232 rows, 7.2 us for
-    // 6.4 + 4.0 us at 61 851 (FP32), but 14.4 us for 9.7 + 4.5 us at 212 117.
+    // 6.2 + 3.1 us; 7 663 rows in CSR take 4.6 us and 3.4 + 3.0 us.
+    // The start from zero reads b and D^-1 where the step alone reads x, so it
+    // costs more per stored entry and saves a launch and a pass.  On first
+    // levels (11 entries a row) it takes 7.9 us for 6.5 + 4.8 us at 114 444 rows
+    // in FP64 (FP32: 6.3 for 5.0 + 4.1), 10.7 for 8.2 + 4.9 at 187 200 (8.5 for
+    // 6.5 + 4.8), 23.7 for 18.9 + 5.5 at 517 440 (18.4 for 12.9 + 5.2); on
+    // second levels, whose rows are longer, 10.9 for 8.1 + 4.7 at 101 300 (8.1
+    // for 6.2 + 4.4) but 15.0 for 11.1 + 3.0 at 142 200 (11.0 for 8.1 + 2.9).  The
+    // line lies below the first level measured that loses.
     if (!agg && A.nbr > 131072) return false;
     if (A.sliced_state == 1 && (A.sliced->kind != 2 || agg)) return false;
     FH_CHECK(xnew != x && xnew != b && d != nullptr && d != x && d != xnew, -3,
