@@ -1,6 +1,8 @@
 """Buffers that the assembly and the condensation take from released ones:
 results do not depend on what such a buffer held before, results that are
 alive keep their values."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -61,6 +63,7 @@ def _used():
 def test_kept_memory_is_bounded_and_released():
     ctx = G.Context(0)
     P = G.HhoProblem(dim=3, mesh="hex", n=20, k=3, perturb=0.15, seed=1, defer_assembly=True)
+    gc.collect()  # nothing of other tests is released meanwhile
     P.assemble_gpu(ctx)  # what the first call sets up for good
     G.release_memory()
     used, total = _used()
